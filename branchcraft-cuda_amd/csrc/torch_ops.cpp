@@ -335,6 +335,35 @@ void copy_pages_hip(at::Tensor& cache_k, at::Tensor& cache_v,
                "copy_pages_");
 }
 
+// A prompt's K and V rows into the pages of a host-side list (the reference
+// copies slice by slice, python/branchcraft_torch/transaction.py:64-81).
+void write_prefix_hip(at::Tensor& cache_k, at::Tensor& cache_v, const at::Tensor& k,
+                      const at::Tensor& v, at::IntArrayRef pages) {
+  check_dev_contig(cache_k, "cache_k", at::kHalf);
+  check_dev_contig(cache_v, "cache_v", at::kHalf);
+  TORCH_CHECK(k.is_cuda() && v.is_cuda() && k.scalar_type() == at::kHalf &&
+                  v.scalar_type() == at::kHalf,
+              "k and v must be GPU FP16 tensors");
+  TORCH_CHECK(cache_k.dim() == 4 && cache_v.sizes() == cache_k.sizes() &&
+                  cache_k.size(1) == BC_PAGE_SIZE && k.dim() == 3 && v.sizes() == k.sizes() &&
+                  k.size(1) == cache_k.size(2) && k.size(2) == cache_k.size(3) &&
+                  k.stride(2) == 1 && v.stride(2) == 1 &&
+                  int64_t(pages.size()) == (k.size(0) + BC_PAGE_SIZE - 1) / BC_PAGE_SIZE,
+              "write_prefix shape mismatch");
+  TORCH_CHECK(cache_k.device() == cache_v.device() && cache_k.device() == k.device() &&
+                  cache_k.device() == v.device(),
+              "all tensors must share a device");
+  const c10::DeviceGuard guard(cache_k.device());
+  c10::SmallVector<int32_t, 512> ids(pages.begin(), pages.end());
+  bc_shape shape{1, int(cache_k.size(2)), int(cache_k.size(2)), int(cache_k.size(3)), 1,
+                 int(cache_k.size(0))};
+  if (k.size(0) == 0) return;
+  check_launch(bc_write_prefix(shape, hptr(k), hptr(v), k.stride(0), k.stride(1), v.stride(0),
+                               v.stride(1), hptr_mut(cache_k), hptr_mut(cache_v), ids.data(),
+                               int(k.size(0)), current_stream()),
+               "write_prefix_");
+}
+
 }  // namespace
 
 TORCH_LIBRARY(branchcraft, m) {
@@ -343,6 +372,7 @@ TORCH_LIBRARY(branchcraft, m) {
   m.def("commit_path_(Tensor(a!) cache_k, Tensor(b!) cache_v, Tensor draft_k, Tensor draft_v, Tensor path_nodes, Tensor dest_pages, Tensor dest_slots, int request) -> ()");
   m.def("copy_pages_(Tensor(a!) cache_k, Tensor(b!) cache_v, Tensor src_pages, Tensor dst_pages) -> ()");
   m.def("commit_paths_(Tensor(a!) cache_k, Tensor(b!) cache_v, Tensor draft_k, Tensor draft_v, Tensor requests, Tensor path_nodes, Tensor dest_pages, Tensor dest_slots) -> ()");
+  m.def("write_prefix_(Tensor(a!) cache_k, Tensor(b!) cache_v, Tensor k, Tensor v, int[] pages) -> ()");
   m.def("paged_decode(Tensor q, Tensor k, Tensor v, Tensor pages, Tensor lengths, int splits=0) -> Tensor");
 }
 
@@ -352,5 +382,6 @@ TORCH_LIBRARY_IMPL(branchcraft, CUDA, m) {
   m.impl("commit_path_", commit_path_hip);
   m.impl("copy_pages_", copy_pages_hip);
   m.impl("commit_paths_", commit_paths_hip);
+  m.impl("write_prefix_", write_prefix_hip);
   m.impl("paged_decode", paged_decode_hip);
 }

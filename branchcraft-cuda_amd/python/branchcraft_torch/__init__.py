@@ -56,6 +56,11 @@ def _fake_commit_paths(cache_k, cache_v, draft_k, draft_v, requests, path_nodes,
     return None
 
 
+@torch.library.register_fake("branchcraft::write_prefix_")
+def _fake_write_prefix(cache_k, cache_v, k, v, pages):
+    return None
+
+
 def tree_verify(q, prefix_k, prefix_v, pages, lengths, draft_k, draft_v, parent):
     """FP32 [batch, node, query head, dim] outputs; every node attends to its
     request's paged prefix and its own ancestor chain (itself included)."""
@@ -101,5 +106,12 @@ def commit_paths_(cache_k, cache_v, draft_k, draft_v, requests, path_nodes, dest
         cache_k, cache_v, draft_k, draft_v, requests, path_nodes, dest_pages, dest_slots)
 
 
+def write_prefix_(cache_k, cache_v, k, v, pages):
+    """Fill the pages of a host-side list with a prompt's K and V rows
+    ([tokens, KV heads, dim], any strides with a contiguous last dim): token t
+    goes to (pages[t // 16], t % 16).  Pages must be distinct."""
+    return torch.ops.branchcraft.write_prefix_(cache_k, cache_v, k, v, pages)
+
+
 __all__ = ["tree_verify", "packed_decode_out", "paged_decode",
-           "commit_path_", "copy_pages_", "commit_paths_", "LIBRARY_PATH"]
+           "commit_path_", "copy_pages_", "commit_paths_", "write_prefix_", "LIBRARY_PATH"]

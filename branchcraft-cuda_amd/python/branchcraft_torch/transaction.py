@@ -17,7 +17,7 @@ from __future__ import annotations
 
 import torch
 
-from . import commit_path_, commit_paths_, copy_pages_, tree_verify
+from . import commit_path_, commit_paths_, copy_pages_, tree_verify, write_prefix_
 from .pages import CommitPlan, PageOwner, Snapshot
 
 __all__ = ["PagedTreeCache", "Snapshot", "CommitPlan"]
@@ -60,11 +60,33 @@ class PagedTreeCache:
             raise ValueError("prefix head shape differs from cache")
         tokens = prefix_k.shape[0]
         request = self.owner.new(tokens)
-        for i, page in enumerate(self.owner.pages[request]):
-            n = min(16, tokens - 16 * i)
+        self._write_prefix(self.owner.pages[request], prefix_k, prefix_v)
+        return request
+
+    def _write_prefix(self, pages: list[int], prefix_k: torch.Tensor,
+                      prefix_v: torch.Tensor) -> None:
+        """Prompt rows into fresh pages: one launch, the page ids in its
+        kernel arguments.  What the op does not take -- a pool that is not on
+        the GPU, rows that autograd tracks, a subclass, or rows that are views
+        of the pool itself -- is copied page by page."""
+        store = [x.untyped_storage().data_ptr() for x in (self.k, self.v)]
+        rows = []
+        for x in (prefix_k, prefix_v):
+            if (not self.k.is_cuda or type(x) not in (torch.Tensor, torch.nn.Parameter)
+                    or (x.requires_grad and torch.is_grad_enabled())
+                    or x.untyped_storage().data_ptr() in store):
+                break
+            # V of another type or device is converted as a copy would.
+            x = x.to(self.k.device, torch.float16)
+            rows.append(x if x.stride(-1) == 1 else x.contiguous())
+        else:
+            if pages:
+                write_prefix_(self.k, self.v, *rows, pages)
+            return
+        for i, page in enumerate(pages):
+            n = min(16, prefix_k.shape[0] - 16 * i)
             self.k[page, :n].copy_(prefix_k[16 * i:16 * i + n])
             self.v[page, :n].copy_(prefix_v[16 * i:16 * i + n])
-        return request
 
     def fork(self, source: int) -> int:
         return self.owner.fork(source)

@@ -224,6 +224,21 @@ int bc_copy_pages(bc_shape shape, bc_half* cache_k, bc_half* cache_v,
                   const int32_t* src_pages, const int32_t* dst_pages,
                   int count, bc_stream_t stream);
 
+/* Fill a request's pages with its prompt's K and V rows: token t of k and v
+ * ([tokens, Hkv, D], strides in elements, the head dimension contiguous) goes
+ * to cache[host_pages[t / 16], t % 16].  host_pages is HOST memory (one id
+ * per started page), read before the call returns: the ids travel in the
+ * kernel arguments, up to 896 pages per launch.  Out-of-range page ids are
+ * skipped as in bc_copy_pages; pages must be distinct and the rows must not
+ * lie in pages being written.  Any 2-byte aligned pointers and any
+ * non-negative strides work.  Replaces the two slice copies per page of
+ * python/branchcraft_torch/transaction.py:64-81. */
+int bc_write_prefix(bc_shape shape, const bc_half* k, const bc_half* v,
+                    long long k_token_stride, long long k_head_stride,
+                    long long v_token_stride, long long v_head_stride,
+                    bc_half* cache_k, bc_half* cache_v,
+                    const int32_t* host_pages, int tokens, bc_stream_t stream);
+
 /* vLLM-style packed-cache decode with FP16 output.  Token t of sequence b
  * lives at element offset
  *   pages[b, t/16]*block_stride + kvh*head_stride + (t%16)*slot_stride

@@ -1,0 +1,86 @@
+"""write_prefix_ and PagedTreeCache.new: a prompt's rows in the pages of a
+host-side list, bit for bit what copying page by page leaves."""
+
+import pytest
+import torch
+
+
+def _by_page(cache, rows, pages):
+    want = cache.clone()
+    for i, p in enumerate(pages):
+        n = min(16, rows.shape[0] - 16 * i)
+        want[p, :n] = rows[16 * i:16 * i + n]
+    return want
+
+
+def _bits(x):
+    return x.contiguous().view(torch.int16)
+
+
+# Tokens at the edges of a slice (4), a page (16) and the ids one launch
+# carries (896 pages), and two launches.
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,hkv,d", [(1, 8, 128), (4, 1, 64), (5, 3, 64), (16, 8, 128),
+                                          (17, 8, 64), (333, 5, 128), (896 * 16, 1, 64),
+                                          (896 * 16 + 5, 2, 64)])
+@pytest.mark.parametrize("form", ["plain", "fused", "heads_first", "unaligned", "expanded"])
+def test_write_prefix_matches_page_copies(tokens, hkv, d, form):
+    import branchcraft_torch as bt
+    torch.manual_seed(tokens + d)
+    count = -(-tokens // 16)
+
+    def half(*shape):
+        return torch.randn(shape, device="cuda", dtype=torch.float16)
+
+    if form == "fused":  # slices of one qkv projection
+        fused = half(tokens, 3, hkv, d)
+        k, v = fused[:, 1], fused[:, 2]
+    elif form == "heads_first":
+        k, v = half(hkv, tokens, d).transpose(0, 1), half(tokens, hkv, d)
+    elif form == "unaligned":
+        k, v = half(tokens * hkv * d + 1)[1:].view(tokens, hkv, d), half(tokens, hkv, d)
+    elif form == "expanded":
+        k, v = half(tokens, 1, d).expand(tokens, hkv, d), half(1, hkv, d).expand(tokens, hkv, d)
+    else:
+        k, v = half(tokens, hkv, d), half(tokens, hkv, d)
+    ck, cv = half(count + 3, 16, hkv, d), half(count + 3, 16, hkv, d)
+    pages = torch.randperm(count + 3)[:count].tolist()
+    want_k, want_v = _by_page(ck, k, pages), _by_page(cv, v, pages)
+    bt.write_prefix_(ck, cv, k, v, pages)
+    assert torch.equal(_bits(ck), _bits(want_k)) and torch.equal(_bits(cv), _bits(want_v))
+
+
+@pytest.mark.gpu
+def test_new_takes_what_the_op_does_not():
+    """V of another type or on the host, a strided last dimension, rows that
+    are views of the pool, rows under autograd and an empty prompt."""
+    from branchcraft_torch.transaction import PagedTreeCache
+    torch.manual_seed(4)
+
+    def check(k, v, store=None):
+        store = store or PagedTreeCache(12, 2, 64)
+        before_k, before_v = store.k.detach().clone(), store.v.detach().clone()
+        pages = store.pages[store.new(k, v)]
+        assert torch.equal(_bits(store.k.detach()), _bits(_by_page(before_k, k.detach(), pages)))
+        assert torch.equal(_bits(store.v.detach()),
+                           _bits(_by_page(before_v, v.detach().to(before_v), pages)))
+        return store
+
+    k = torch.randn(37, 2, 64, device="cuda", dtype=torch.float16)
+    check(k, torch.randn(37, 2, 64, device="cuda"))
+    check(k, torch.randn(37, 2, 64, dtype=torch.float16))
+    check(torch.randn(37, 64, 2, device="cuda", dtype=torch.float16).transpose(1, 2), k)
+    check(k[:0], k[:0])
+    assert check(k.clone().requires_grad_(), k).k.requires_grad
+    store = check(k, k)
+    check(store.k[:2].view(32, 2, 64), store.v[:2].view(32, 2, 64), store)
+
+
+def test_new_on_a_host_pool_copies_by_page():
+    pytest.importorskip("branchcraft_torch")
+    from branchcraft_torch.transaction import PagedTreeCache
+    store = PagedTreeCache(5, 2, 64, device="cpu")
+    k, v = (torch.randn(19, 2, 64).half() for _ in range(2))
+    pages = store.pages[store.new(k, v)]
+    assert torch.equal(store.k, _by_page(torch.zeros_like(store.k), k, pages))
+    assert torch.equal(store.v, _by_page(torch.zeros_like(store.v), v, pages))
