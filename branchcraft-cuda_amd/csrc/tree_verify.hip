@@ -29,11 +29,12 @@
 //    four waves each on the same tiles.  Workgroup ids put
 //    (KV head, row tile) in the low bits, so requests that share prefix
 //    pages run on the same XCD and reuse its L2.
-//  - tree_rows_kernel: trees of many row tiles per (request, KV head), whose
-//    units already fill the CUs: four waves take four row tiles and walk the
-//    same K/V tiles, loaded once per workgroup.
-//  - tree_kernel: the single pass for tensors that are not 16-byte aligned
-//    (element-wise loads and stores).
+//  - tree_wide_kernel: trees of several row tiles per (request, KV head): four
+//    waves take four row tiles (or two, two waves each) and share K/V tiles
+//    that are loaded straight into LDS, whole prefixes or parts of them.
+//  - tree_rows_kernel, tree_kernel: element-wise loads and stores, for tensors
+//    that are not 16-byte aligned (and, tree_kernel, calls without the pool
+//    size): a K/V tile shared by four row tiles, and one row tile each.
 #include <type_traits>
 
 #include "bc_device.h"
@@ -1186,15 +1187,471 @@ void launch_merge_split(const TreeParams& P, dim3 grid, hipStream_t st) {
   else merge_split_kernel<D, 4><<<grid, 256, 0, st>>>(P);
 }
 
-// Row-sharing variant for trees of four or more row tiles per (request, KV
-// head), where tree_kernel would read the prefix once per row tile: the four
+// ---- softmax pieces of tree_wide_kernel ----
+
+// Scores of the lane's query row at the tokens outside ok to -inf: sc[j] holds
+// token row 8*(j/4) + 4*g + j%4.
+__device__ __forceinline__ void row_mask(f32x16& sc, uint32_t ok, int g) {
+  const uint32_t ob = ok >> (4 * g);
+#pragma unroll
+  for (int j = 0; j < 16; ++j) sc[j] = (ob >> (8 * (j >> 2) + (j & 3))) & 1u ? sc[j] : kNegInf;
+}
+
+// Online softmax: moves the row's running max m (log2 units) for the raw
+// scores of NT tiles and rescales l and acc.  The max moves only when it
+// would grow by more than kRescaleSlack, so the two lane halves of a row
+// compare their own maxima and exchange them only then.
+template <int DT, int NT>
+__device__ __forceinline__ void row_max(const f32x16 (&sc)[NT], float scale_log2, float& m,
+                                         float& l, f32x16 (&acc)[DT]) {
+  float tmax = kNegInf;
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) tmax = __builtin_fmaxf(tmax, sc[i][j]);
+  tmax *= scale_log2;
+  if (__builtin_amdgcn_ballot_w64(tmax > m + kRescaleSlack)) {
+    const float mnew = __builtin_fmaxf(m, __builtin_fmaxf(tmax, shfl_xor_f(tmax, 32)));
+    const float alpha = fast_exp2(m - safe_max(mnew));
+    l *= alpha;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) acc[dt][j] *= alpha;
+    m = mnew;
+  }
+}
+
+// Weights of the 16 tokens 16 half .. of a tile as an FP16 hi/lo pair (see
+// split_hi_lo), added to l; mb is the exponent base.
+__device__ __forceinline__ void row_weights(const f32x16& sc, int half, float scale_log2,
+                                             float mb, float& l, f16x8& pb, f16x8& pl) {
+  uint32_t wh[4], wl[4];
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    const float p0 = fast_exp2(__builtin_fmaf(sc[8 * half + 2 * x], scale_log2, -mb));
+    const float p1 = fast_exp2(__builtin_fmaf(sc[8 * half + 2 * x + 1], scale_log2, -mb));
+    l += p0;
+    l += p1;
+    split_hi_lo(p0, p1, wh[x], wl[x]);
+  }
+  pb = __builtin_bit_cast(f16x8, u32x4{wh[0], wh[1], wh[2], wh[3]});
+  pl = __builtin_bit_cast(f16x8, u32x4{wl[0], wl[1], wl[2], wl[3]});
+}
+
+// 16-byte chunk c of token row `row` sits at chunk c ^ swz<D>(row) of the
+// row's place in LDS: rows need no padding (a load straight into LDS fills
+// consecutive lanes' chunks), and both the K reads (16 rows, one chunk each)
+// and the V transpose reads (four rows, four chunks each) touch every bank
+// once.
+template <int D>
+__device__ __forceinline__ int swz(int row) {
+  return D == 128 ? ((row & 3) << 2) | ((row >> 2) & 3) : (((row >> 1) & 1) << 2) | ((row >> 2) & 3);
+}
+
+// 16 bytes per lane straight into LDS, lane i's at dst + 16 i (dst
+// wave-uniform).  No register waits for it: the caller waits with
+// wait_loads() before the barrier that publishes the data.
+__device__ __forceinline__ void load_to_lds(const void* src, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+               :
+               : "v"(src), "s"(dst)
+               : "memory");
+}
+
+__device__ __forceinline__ void load_to_lds(const void* base, unsigned off, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :
+               : "v"(off), "s"(base), "s"(dst)
+               : "memory");
+}
+
+__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Wide trees: a workgroup takes RT row tiles of one (request, KV head) and
+// part `part` of its steps (two 32-token tiles each: draft tiles first, then
+// prefix tiles), which its four waves share through LDS, 4 / RT waves on each
+// row tile: with RT = 4 a wave takes both tiles of a step, with RT = 2 one.
+// Each step's K and V go straight into the other of two LDS buffers while
+// the current one is computed, one barrier per step, and hold no registers,
+// so the reads of a whole step's K can be in flight at once.  With one part
+// the rows go to the output, else each part leaves an FP32 partial in slot
+// (row, part) for merge_split_kernel.
+// Bound by the matrix units and their clock: 8 requests x 2048 tokens x 256
+// nodes (32/8 heads, D = 128) take 116 us, 594 TFLOP/s (891 with the second
+// MFMA that P's low part takes); the MFMAs alone fill half the cycles, and
+// the clock falls from 2.4 to 1.8 GHz under them.  One 32-token tile per
+// barrier, staged through registers, took 143 us.
+template <int D, int RT>
+__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreeParams P) {
+  constexpr int KS = D / 16;      // MFMA k-steps over the head dimension
+  constexpr int DT = D / 32;      // 32-row output tiles over the head dimension
+  constexpr int TPS = 2;          // tiles per step
+  constexpr int TS = 4 / RT;      // waves per row tile
+  constexpr int TPW = TPS / TS;   // tiles per wave and step
+  static_assert(TPW >= 1, "RT is 2 or 4");
+  constexpr int CPR = D / 8;      // 16-byte chunks per token row
+  constexpr int CPT = kTile * CPR / 256;  // chunks per thread and tile, K and V each
+  constexpr int HALF = kTile * D;   // halves of a tile's K (then as many of V)
+  constexpr int TILE = 2 * HALF;
+  constexpr int PPS = TPS * kTile / BC_PAGE_SIZE;  // pages per step
+  constexpr int SPC = 64 / PPS;                    // steps per register of page ids
+
+  pin_params(P);
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 5;   // lane half
+  const int lr = lane & 31;  // tile column (query row) / token slot
+  const int wrt = wave % RT, wts = wave / RT;  // this wave's row tile and tile of a step
+
+  __shared__ __attribute__((aligned(256))) _Float16 s_kv[2][TPS * TILE];
+  __shared__ uint4 s_anc[BC_MAX_TREE_NODES][2];  // ancestor-or-self set per node, 256 bits
+  __shared__ int s_ptr[BC_MAX_TREE_NODES];
+
+  // Workgroup ids put (KV head, row group) in the low bits, then the request,
+  // then the part.
+  const int rgroups = (P.row_tiles + RT - 1) / RT;
+  const int zdim = P.hkv * rgroups;
+  const int unit = blockIdx.x % (zdim * P.batch), part = blockIdx.x / (zdim * P.batch);
+  const int z = unit % zdim, b = unit / zdim;
+  const int kvh = z / rgroups;
+  const int t0 = part * (P.tiles_per_part / TPS);
+
+  // First round of loads: the page ids (lane i of a register: entry i of the
+  // 64 table entries from step t on, from inside the request's table row),
+  // the row's Q^T fragments (rows past the tree read row (node 0, head 0),
+  // whose columns are never written out), the parents and the length.
+  const int ntd = (P.nodes + kTile - 1) / kTile;
+  auto load_ids = [&](int t) {
+    const int pg = t * PPS - ntd * (kTile / BC_PAGE_SIZE) + lane;
+    return P.pages[(size_t)b * P.max_pages + min(max(pg, 0), P.max_pages - 1)];
+  };
+  int ids = load_ids(t0), ids_next = load_ids(t0 + SPC);
+  const int r = ((z - kvh * rgroups) * RT + wrt) * 32 + lr;
+  const int rnode = div_by(r, P.group, P.group_mul);
+  const int node = r < P.rows ? rnode : 0;
+  const int h = kvh * P.group + (r < P.rows ? r - rnode * P.group : 0);
+  uint4 qB[KS];
+  {
+    const uint16_t* qp = P.dq + (((size_t)b * P.nodes + node) * P.hq + h) * D + 8 * g;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qB[s] = ldg16(qp + 16 * s);
+  }
+  const int me = min(tid, P.nodes - 1);
+  int up = P.parent[(size_t)b * P.nodes + me];
+  const int len = max(0, min(P.lengths[b], P.max_pages * BC_PAGE_SIZE));
+  const int ntile = ntd + (len + kTile - 1) / kTile;
+  const int tend = min((ntile + TPS - 1) / TPS, t0 + P.tiles_per_part / TPS);
+  if (t0 >= tend) return;  // uniform: the request ends before this part
+
+  // Loads: chunk c of a tile is token row (tid + 256c) / CPR, 16 bytes at
+  // 8 * (tid % CPR); a wave's chunk lies in one page.
+  const int lrow = tid / CPR, lcol = 8 * (tid % CPR ^ swz<D>(lrow));
+  const size_t tok_stride = (size_t)P.hkv * D;
+  const unsigned loff = (unsigned)(((lrow % BC_PAGE_SIZE) * tok_stride + lcol) * sizeof(uint16_t));
+  const unsigned page_bytes = (unsigned)(BC_PAGE_SIZE * tok_stride * sizeof(uint16_t));
+  const char* const kb = reinterpret_cast<const char*>(P.k + (size_t)kvh * D);
+  const char* const vb = reinterpret_cast<const char*>(P.v + (size_t)kvh * D);
+  // LDS byte address of this wave's first chunk of tile 0's K in buffer 0.
+  const unsigned lds0 = __builtin_amdgcn_readfirstlane(
+      (unsigned)(uintptr_t)(__attribute__((address_space(3))) _Float16*)s_kv + wave * 1024);
+  auto lds_of = [&](int buf, int i, int c) {
+    return lds0 + (unsigned)(buf * TPS * TILE * 2 + i * TILE * 2 + c * 4096);
+  };
+  // Chunk x of a prefix step from page ids inside the pool, K and V.
+  constexpr int NX = TPS * CPT;
+  auto issue_chunk = [&](int x, const int (&ph)[PPS], int buf) {
+    const int i = x / CPT, c = x % CPT;
+    const unsigned id = CPT == 2 ? ph[2 * i + c] : wave < 2 ? ph[2 * i] : ph[2 * i + 1];
+    const unsigned long long off = (unsigned long long)id * page_bytes;
+    load_to_lds(kb + off, loff, lds_of(buf, i, c));
+    load_to_lds(vb + off, loff, lds_of(buf, i, c) + HALF * 2);
+  };
+  // Any step.  Pages outside the pool read page 0, rows past the length
+  // their page's rows and draft rows past the node count the last node's: all
+  // in bounds, all masked (a draft tile's page ids are unused).
+  auto issue = [&](int t, const int (&ph)[PPS], int buf) {
+    int in[PPS];
+#pragma unroll
+    for (int q = 0; q < PPS; ++q) in[q] = (unsigned)ph[q] < (unsigned)P.phys_pages ? ph[q] : 0;
+#pragma unroll
+    for (int x = 0; x < NX; ++x) {
+      const int i = x / CPT, c = x % CPT, it = t * TPS + i;
+      if (it >= ntd) {
+        issue_chunk(x, in, buf);
+      } else {
+        const int dn = min(it * kTile + lrow + 256 / CPR * c, P.nodes - 1);
+        const size_t off = (((size_t)b * P.nodes + dn) * P.hkv + kvh) * D + lcol;
+        load_to_lds(P.dk + off, lds_of(buf, i, c));
+        load_to_lds(P.dv + off, lds_of(buf, i, c) + HALF * 2);
+      }
+    }
+  };
+  // Whether every token of the step is a valid prefix token; else the valid
+  // ones per tile (of draft tiles: of the node count) in rows.
+  auto whole_step = [&](int t, const int (&ph)[PPS], uint32_t (&rows)[TPS]) {
+    bool ok = t * TPS >= ntd && ((t + 1) * TPS - ntd) * kTile <= len;
+#pragma unroll
+    for (int q = 0; q < PPS; ++q) ok = ok && (unsigned)ph[q] < (unsigned)P.phys_pages;
+    if (ok) return true;
+#pragma unroll
+    for (int i = 0; i < TPS; ++i) {
+      const int it = t * TPS + i;
+      rows[i] = __builtin_amdgcn_readfirstlane(
+          it < ntd ? prefix_bits(P.nodes - it * kTile, 0, 0, 1)
+                   : prefix_bits(len - (it - ntd) * kTile, ph[2 * i], ph[2 * i + 1], P.phys_pages));
+    }
+    return false;
+  };
+  // V rows that are not valid tokens may hold any bits (NaN included): their
+  // weight is zero, so the rows must be zero.  Each lane clears the chunks
+  // that its own loads, already waited for, have filled.
+  auto clear = [&](const uint32_t (&rows)[TPS], _Float16* buf) {
+#pragma unroll
+    for (int i = 0; i < TPS; ++i)
+#pragma unroll
+      for (int c = 0; c < CPT; ++c)
+        if (!((rows[i] >> (lrow + 256 / CPR * c)) & 1u))
+          *reinterpret_cast<uint4*>(buf + i * TILE + HALF + (tid + 256 * c) * 8) =
+              make_uint4(0, 0, 0, 0);
+  };
+  auto take_ids = [&](int v, int step, int (&ph)[PPS]) {
+#pragma unroll
+    for (int q = 0; q < PPS; ++q) ph[q] = __builtin_amdgcn_readlane(v, step * PPS + q);
+  };
+
+  int ph[PPS];
+  uint32_t rows[TPS] = {~0u, ~0u};
+  take_ids(ids, 0, ph);
+  issue(t0, ph, 0);
+  bool whole = whole_step(t0, ph, rows);
+
+  // Ancestor sets, while the first step loads.  Pointer doubling: after round
+  // k thread i holds the nodes within 2^k steps of node i and the node 2^k
+  // steps up, so a chain of any depth (or a cycle) takes at most eight
+  // rounds; a serial walk pays one LDS round trip per step of the chain, in
+  // every draft tile (2 requests x 333 tokens x a 256-node chain: 88.6 us).
+  if (t0 * TPS < ntd) {  // uniform: the part holds draft tiles
+    uint32_t set[8];
+#pragma unroll
+    for (int w = 0; w < 8; ++w) set[w] = (me >> 5) == w ? 1u << (me & 31) : 0u;
+    if (up < 0 || up >= P.nodes) up = -1;
+    for (int round = 0;; ++round) {
+      s_anc[tid][0] = make_uint4(set[0], set[1], set[2], set[3]);
+      s_anc[tid][1] = make_uint4(set[4], set[5], set[6], set[7]);
+      s_ptr[tid] = up;
+      if (!__syncthreads_or(up >= 0) || round == 8) break;  // uniform
+      if (up >= 0) {
+        const uint4 s0 = s_anc[up][0], s1 = s_anc[up][1];
+        set[0] |= s0.x;
+        set[1] |= s0.y;
+        set[2] |= s0.z;
+        set[3] |= s0.w;
+        set[4] |= s1.x;
+        set[5] |= s1.y;
+        set[6] |= s1.z;
+        set[7] |= s1.w;
+        up = s_ptr[up];
+      }
+      __syncthreads();
+    }
+  }
+
+  // Read offsets in a staged tile (halves): K chunk 2s + g of row lr, and the
+  // V transpose reads' [token 4 * (trG / 2) + trj / 4 (+ 8 hf)][dim
+  // 16 * (trG % 2) + 4 * (trj % 4) (+ 32 dt)].
+  const int trG = lane >> 4, trj = lane & 15;
+  int koff[KS], voff[2][DT];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) koff[s] = lr * D + ((2 * s + g) ^ swz<D>(lr)) * 8;
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      const int row = 4 * (trG >> 1) + (trj >> 2) + 8 * hf;
+      const int dim = 32 * dt + 16 * (trG & 1) + 4 * (trj & 3);
+      voff[hf][dt] = HALF + row * D + ((dim >> 3) ^ swz<D>(row)) * 8 + (dim & 7);
+    }
+  f32x16 acc[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[dt][j] = 0.f;
+  float m = kNegInf, l = 0.f;
+  constexpr int NG = 2 * TPW;  // 16-token groups per wave and step
+  static_assert(KS / 2 >= NX, "a step's loads fit between its score MFMAs");
+  // The wait for Q belongs here: left to its first use, inside the step
+  // loop, the compiler's wait there also covers the loads each step has just
+  // issued.
+#pragma unroll
+  for (int s = 0; s < KS; ++s)
+    asm volatile("" : "+v"(qB[s].x), "+v"(qB[s].y), "+v"(qB[s].z), "+v"(qB[s].w));
+  wait_loads();
+  if (!whole) clear(rows, s_kv[0]);
+  __syncthreads();
+
+  int k = 0;
+  for (int t = t0; t < tend; ++t) {
+    // The next step's page ids; a step of other than valid prefix tokens
+    // only is issued here, the others between the score MFMAs below: issued
+    // together, the four waves' loads queue for the CU's 64 bytes per clock
+    // and hold up the math behind them.
+    bool whole_n = true, next = false;
+    uint32_t rows_n[TPS] = {~0u, ~0u};
+    if (t + 1 < tend) {
+      const int i = (t + 1 - t0) % SPC;
+      if (i == 0) {
+        ids = ids_next;
+        ids_next = load_ids(t + 1 + SPC);
+      }
+      take_ids(ids, i, ph);
+      whole_n = next = whole_step(t + 1, ph, rows_n);
+      if (!next) issue(t + 1, ph, k ^ 1);
+    }
+    const _Float16* base = s_kv[k] + (TS == 1 ? 0 : wts * TILE);
+    f16x8 kf[TPW][KS], av[2][DT];
+    f32x16 sc[TPW];
+    auto read_v = [&](int grp) {
+      const _Float16* v0 = base + grp / 2 * TILE + grp % 2 * 16 * D;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const f16x4 lo = lds_read_tr(v0 + voff[0][dt]);
+        const f16x4 hi = lds_read_tr(v0 + voff[1][dt]);
+        av[grp % 2][dt] = f16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      }
+    };
+    // ---- S^T = K Q^T ----
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int i = 0; i < TPW; ++i)
+        kf[i][s] = as_f16x8(*reinterpret_cast<const uint4*>(base + i * TILE + koff[s]));
+#pragma unroll
+    for (int i = 0; i < TPW; ++i)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) sc[i][j] = 0.f;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+#pragma unroll
+      for (int i = 0; i < TPW; ++i)
+        sc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[i][s], as_f16x8(qB[s]), sc[i], 0, 0, 0);
+      if (s % 2 == 1 && s / 2 < NX) {
+        if (next) issue_chunk(s / 2, ph, k ^ 1);  // uniform
+      }
+    }
+    // ---- mask and online softmax (column lr = query row) ----
+    if (!whole) {
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+        const int it = t * TPS + (TS == 1 ? i : wts);
+        const uint32_t ok = it < ntd ? reinterpret_cast<const uint32_t*>(s_anc[node])[it]
+                                     : TS == 1 ? rows[i] : wts ? rows[1] : rows[0];
+        row_mask(sc[i], ok, g);
+      }
+    }
+    row_max<DT, TPW>(sc, P.scale_log2, m, l, acc);
+    // ---- O^T += V^T P^T, the next group's weights between the MFMAs ----
+    const float mb = safe_max(m);
+    f16x8 pb[2], pl[2];
+    auto weights = [&](int grp) {
+      row_weights(sc[grp / 2], grp % 2, P.scale_log2, mb, l, pb[grp % 2], pl[grp % 2]);
+    };
+    read_v(0);
+    weights(0);
+#pragma unroll
+    for (int grp = 0; grp < NG; ++grp) {
+      if (grp + 1 < NG) {
+        read_v(grp + 1);
+        weights(grp + 1);
+      }
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+        acc[dt] =
+            __builtin_amdgcn_mfma_f32_32x32x16_f16(av[grp % 2][dt], pb[grp % 2], acc[dt], 0, 0, 0);
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+        acc[dt] =
+            __builtin_amdgcn_mfma_f32_32x32x16_f16(av[grp % 2][dt], pl[grp % 2], acc[dt], 0, 0, 0);
+    }
+    wait_loads();
+    if (!whole_n) clear(rows_n, s_kv[k ^ 1]);
+    __syncthreads();
+    k ^= 1;
+    whole = whole_n;
+#pragma unroll
+    for (int i = 0; i < TPS; ++i) rows[i] = rows_n[i];
+  }
+
+  // ---- the rows' output, or this part's partial of them ----
+  l += shfl_xor_f(l, 32);  // both lane halves share m
+  if constexpr (TS > 1) {
+    // The waves of a row tile merge through LDS (every staged tile has been
+    // read).  Four-float chunk c of row lr sits at c ^ (lr % (D / 4)), so an
+    // access of 32 rows spreads over the banks; (max, sum) go to s_ptr.
+    static_assert(RT * 32 * D * 4 <= TPS * TILE * 2, "the states fit one buffer");
+    static_assert(RT * 64 <= BC_MAX_TREE_NODES, "(max, sum) pairs fit s_ptr");
+    float* mine = reinterpret_cast<float*>(s_kv[0]) + wrt * 32 * D + lr * D;
+    float2* mine_ml = reinterpret_cast<float2*>(s_ptr) + wrt * 32 + lr;
+    auto at = [&](int d) { return mine + (((d >> 2) ^ (lr % (D / 4))) << 2); };
+    if (wts == 1) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int jq = 0; jq < 4; ++jq)
+          *reinterpret_cast<float4*>(at(32 * dt + 8 * jq + 4 * g)) =
+              make_float4(acc[dt][4 * jq], acc[dt][4 * jq + 1], acc[dt][4 * jq + 2],
+                          acc[dt][4 * jq + 3]);
+      if (g == 0) *mine_ml = make_float2(m, l);
+    }
+    __syncthreads();
+    if (wts == 1) return;
+    const float2 ml = *mine_ml;
+    const float mm = __builtin_fmaxf(m, ml.x);
+    const float a1 = fast_exp2(m - safe_max(mm)), a2 = fast_exp2(ml.x - safe_max(mm));
+    l = l * a1 + ml.y * a2;
+    m = mm;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq) {
+        const float4 v4 = *reinterpret_cast<const float4*>(at(32 * dt + 8 * jq + 4 * g));
+        acc[dt][4 * jq] = acc[dt][4 * jq] * a1 + v4.x * a2;
+        acc[dt][4 * jq + 1] = acc[dt][4 * jq + 1] * a1 + v4.y * a2;
+        acc[dt][4 * jq + 2] = acc[dt][4 * jq + 2] * a1 + v4.z * a2;
+        acc[dt][4 * jq + 3] = acc[dt][4 * jq + 3] * a1 + v4.w * a2;
+      }
+  }
+  if (r >= P.rows) return;
+  const size_t orow = ((size_t)b * P.nodes + node) * P.hq + h;
+  float* dst = P.out + orow * D;
+  float inv = 1.f;
+  if (P.parts == 1) {
+    inv = 1.f / l;  // every row sees its own node: l > 0
+  } else {
+    const size_t slot = orow * P.parts + part;
+    dst = P.part_acc + slot * D;
+    if (g == 0) *reinterpret_cast<float2*>(P.part_ml + 2 * slot) = make_float2(m, l);
+  }
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int jq = 0; jq < 4; ++jq)
+      *reinterpret_cast<float4*>(dst + 32 * dt + 8 * jq + 4 * g) =
+          make_float4(acc[dt][4 * jq] * inv, acc[dt][4 * jq + 1] * inv,
+                      acc[dt][4 * jq + 2] * inv, acc[dt][4 * jq + 3] * inv);
+}
+
+// Row-sharing variant, for tensors that are not 16-byte aligned, of trees of
+// four or more row tiles per (request, KV head), where tree_kernel would read
+// the prefix once per row tile: the four
 // waves take four row tiles and walk the same 32-token tiles, which the
 // workgroup loads once (two 16-byte chunks of K and of V per thread) into a
 // double-buffered LDS tile, one barrier per tile.  Each wave reads K back in
 // the A-operand layout and V through transpose reads, and owns its rows to
 // the end: no merge between waves.  Masks, softmax and the P.V product are
 // those of tree_kernel.
-template <int D, bool VEC>
+template <int D>
 __global__ __launch_bounds__(kThreads, 2) void tree_rows_kernel(TreeParams P) {
   // No pin_params here: this kernel's loop runs tens to hundreds of us, and
   // holding every argument in registers from the start measured 0.4-2%
@@ -1239,7 +1696,7 @@ __global__ __launch_bounds__(kThreads, 2) void tree_rows_kernel(TreeParams P) {
   {
     const uint16_t* qp = P.dq + (((size_t)b * P.nodes + node) * P.hq + h) * D + 8 * g;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) qB[s] = rvalid ? load8<VEC>(qp + 16 * s) : make_uint4(0, 0, 0, 0);
+    for (int s = 0; s < KS; ++s) qB[s] = rvalid ? load8<false>(qp + 16 * s) : make_uint4(0, 0, 0, 0);
   }
   static_assert(BC_MAX_TREE_NODES <= kThreads, "one parent entry per thread");
   const bool has_parent = (int)threadIdx.x < P.nodes;
@@ -1277,14 +1734,14 @@ __global__ __launch_bounds__(kThreads, 2) void tree_rows_kernel(TreeParams P) {
         ok = pok && t < len;
         off = (pok ? ((size_t)pgq * BC_PAGE_SIZE + row % BC_PAGE_SIZE) * tok_stride : 0) +
               (size_t)kvh * D + col;
-        kreg[set][c] = load8<VEC>(P.k + off);
-        vreg[set][c] = load8<VEC>(P.v + off);
+        kreg[set][c] = load8<false>(P.k + off);
+        vreg[set][c] = load8<false>(P.v + off);
       } else {
         const int dn = tbase + row;
         ok = dn < P.nodes;
         off = (((size_t)b * P.nodes + min(dn, P.nodes - 1)) * P.hkv + kvh) * D + col;
-        kreg[set][c] = load8<VEC>(P.dk + off);
-        vreg[set][c] = load8<VEC>(P.dv + off);
+        kreg[set][c] = load8<false>(P.dk + off);
+        vreg[set][c] = load8<false>(P.dv + off);
       }
       vok[set][c] = ok;
     }
@@ -1451,19 +1908,22 @@ __global__ __launch_bounds__(kThreads, 2) void tree_rows_kernel(TreeParams P) {
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int jq = 0; jq < 4; ++jq)
-      store4f<VEC>(dst + 32 * dt + 8 * jq + 4 * g, acc[dt][4 * jq] * inv,
+      store4f<false>(dst + 32 * dt + 8 * jq + 4 * g, acc[dt][4 * jq] * inv,
                    acc[dt][4 * jq + 1] * inv, acc[dt][4 * jq + 2] * inv,
                    acc[dt][4 * jq + 3] * inv);
 }
 
 // The reference's rules (src/tree_attention.cu:94-99): physical_pages is not
 // among them, and a value below 1 means the pool size is not given.
-bool tree_args_ok(const bc_shape& s, const bc_tree_inputs& in, int nodes) {
+bool tree_shape_ok(const bc_shape& s, int nodes) {
   return s.batch >= 1 && s.query_heads >= 1 && s.kv_heads >= 1 &&
          s.query_heads % s.kv_heads == 0 && (s.dim == 64 || s.dim == 128) &&
-         s.max_pages >= 1 && nodes >= 1 && nodes <= BC_MAX_TREE_NODES && in.prefix.k &&
-         in.prefix.v && in.prefix.pages && in.prefix.lengths && in.draft_q && in.draft_k &&
-         in.draft_v && in.parent && in.output;
+         s.max_pages >= 1 && nodes >= 1 && nodes <= BC_MAX_TREE_NODES;
+}
+
+bool tree_args_ok(const bc_shape& s, const bc_tree_inputs& in, int nodes) {
+  return tree_shape_ok(s, nodes) && in.prefix.k && in.prefix.v && in.prefix.pages &&
+         in.prefix.lengths && in.draft_q && in.draft_k && in.draft_v && in.parent && in.output;
 }
 
 // With the pool size given, ids outside [0, physical_pages) are masked and
@@ -1512,46 +1972,18 @@ TreeParams make_params(const bc_shape& s, const bc_tree_inputs& in, int nodes) {
   return P;
 }
 
-// tree_rows_kernel (one K/V tile shared by four row tiles) pays once its
-// row groups fill the CUs: the split kernel would then run several rounds
-// of workgroups that each read the prefix for one row tile (8 requests x
-// 2048 tokens x 256 nodes: 153 against 206 us; 32 x 512 x 64 nodes: 48
-// against 78 us).  With fewer row groups the split kernel wins (8 x 2048 x
-// 64 nodes: 50 against 59 us; 4 x 2048 x 128: 52 against 58 us), and with
-// fewer than four row tiles the rows kernel's serial walk lost outright
-// (one request, 32 nodes: 101 against 36 us).
-bool rows_kernel_for(int batch, int hkv, int row_tiles, int cus) {
-  return row_tiles >= kWaves &&
-         (long long)batch * hkv * ((row_tiles + kWaves - 1) / kWaves) >= cus;
-}
-
-// Workgroups per (request, KV head).
-int row_units(int row_tiles, bool rows_kernel) {
-  return rows_kernel ? (row_tiles + kWaves - 1) / kWaves : row_tiles;
-}
-
-template <int D, bool VEC>
-void launch_tree_kernel(const TreeParams& P, bool rows_kernel, dim3 grid, hipStream_t st) {
-  if (rows_kernel)
-    tree_rows_kernel<D, VEC><<<grid, kThreads, 0, st>>>(P);
-  else  // unaligned tensors or an unknown pool size: the split kernel takes the rest
-    tree_kernel<D, false><<<grid, kThreads, 0, st>>>(P);
-}
-
-// vec: every FP16 tensor and the output are 16-byte aligned (16-byte loads
-// and stores); otherwise the kernels move single halves and floats.
-// known_pool: false sends every shape to tree_kernel (see pool_known).
-hipError_t launch_tree(const TreeParams& P, int dim, bool vec, bool known_pool,
-                       hipStream_t st) {
-  const bool rows_kernel =
-      known_pool && rows_kernel_for(P.batch, P.hkv, P.row_tiles, bch::device_cus());
-  const dim3 grid((unsigned)((size_t)P.batch * P.hkv * row_units(P.row_tiles, rows_kernel)));
-  if (dim == 64) {
-    if (vec) launch_tree_kernel<64, true>(P, rows_kernel, grid, st);
-    else launch_tree_kernel<64, false>(P, rows_kernel, grid, st);
+// Tensors that are not 16-byte aligned, and calls without the pool size:
+// element-wise loads and stores.  tree_rows_kernel (one K/V tile shared by
+// four row tiles) pays once its row groups fill the CUs.
+hipError_t launch_tree(const TreeParams& P, int dim, bool known_pool, hipStream_t st) {
+  const size_t groups = (size_t)P.batch * P.hkv * ((P.row_tiles + kWaves - 1) / kWaves);
+  if (known_pool && P.row_tiles >= kWaves && groups >= (size_t)bch::device_cus()) {
+    if (dim == 64) tree_rows_kernel<64><<<dim3((unsigned)groups), kThreads, 0, st>>>(P);
+    else tree_rows_kernel<128><<<dim3((unsigned)groups), kThreads, 0, st>>>(P);
   } else {
-    if (vec) launch_tree_kernel<128, true>(P, rows_kernel, grid, st);
-    else launch_tree_kernel<128, false>(P, rows_kernel, grid, st);
+    const dim3 grid((unsigned)((size_t)P.batch * P.hkv * P.row_tiles));
+    if (dim == 64) tree_kernel<64, false><<<grid, kThreads, 0, st>>>(P);
+    else tree_kernel<128, false><<<grid, kThreads, 0, st>>>(P);
   }
   return hipGetLastError();
 }
@@ -1562,14 +1994,61 @@ bool tree_ptrs_aligned(const bc_tree_inputs& in) {
          aligned16(in.draft_v) && aligned16(in.output);
 }
 
-// ---- tree_split_kernel: plan, workspace and launch ----
+// ---- aligned tensors: plan, workspace and launch ----
 
 struct SplitPlan {
   int parts;  // workgroups per (request group, KV head, row tile), <= 64
   int tiles;  // 32-token tiles per workgroup and request (draft then prefix tiles)
   int waves;  // waves per workgroup: 4 or 8
   int rq = 1;  // requests per workgroup (waves / rq per request)
+  int wide = 0;  // row tiles per workgroup of tree_wide_kernel (0: tree_split_kernel)
 };
+
+// Units (request, KV head, group of `rt` row tiles) of a launch.
+long long row_groups(const bc_shape& s, int row_tiles, int rt) {
+  return (long long)s.batch * s.kv_heads * ((row_tiles + rt - 1) / rt);
+}
+
+// tree_wide_kernel reads a K/V tile once for four row tiles (or two), where
+// tree_split_kernel reads it per row tile, so it takes the trees of several
+// row tiles whose groups fill the CUs (same box, 32/8 heads and D = 128 unless
+// noted, tree_split_kernel or the kernel it replaced first):
+//  - four row tiles a workgroup from 7/8 CUs of groups on: 8 requests x 2048
+//    tokens x 256 nodes 143 against 116 us, 16 x 1000 x 64 nodes 57 against
+//    40, 64 x 30-500 x 64 nodes 73 against 64, 28/4 heads and D = 64: 64 x
+//    1024 x 128 nodes 137 against 118;
+//  - else two a workgroup from two groups per CU on: 64 x 1024 x 9 nodes 50
+//    against 35 us; and from one group per CU on where the prefixes are not
+//    short (30 tiles): 16/16 heads, D = 64: 16 x 1000 x 33 nodes 25 against
+//    20 us, while 28/4 heads, D = 64, 64 x 30-500 x 9 nodes would take 13.2
+//    against 11.2;
+//  - long prefixes (60 tiles) split into parts, two workgroups per CU, from
+//    5/8 CUs of groups on (D = 64, whose tiles are half as long: one): 8 x
+//    128-4096 x 64 nodes 102 against 63 us, 32 x 256-2048 x 16 nodes 59
+//    against 50.  Fewer groups leave each part too few steps to pay for its
+//    partial rows (8 x 2048 x 64 nodes, 16/2 heads: 26 against 31 us).
+SplitPlan wide_plan(const bc_shape& s, int row_tiles, int max_tiles, int cus) {
+  SplitPlan p{0, 0, 4};
+  if (row_tiles < 2) return p;
+  const int steps = (max_tiles + 1) / 2;
+  p.parts = 1;
+  p.tiles = 2 * steps;
+  p.wide = 4;
+  if (row_tiles > 2 && 8 * row_groups(s, row_tiles, 4) >= 7LL * cus) return p;
+  const long long u = row_groups(s, row_tiles, 2);
+  p.wide = 2;
+  if (u >= 2LL * cus) return p;
+  if (max_tiles >= 60 && 8 * u >= (s.dim == 64 ? 8LL : 5LL) * cus) {
+    const int parts = (int)(2LL * cus / u);  // 1 to 3
+    const int per = (steps + parts - 1) / parts;
+    p.parts = (steps + per - 1) / per;
+    p.tiles = 2 * per;
+    return p;
+  }
+  if (max_tiles >= 30 && u >= cus) return p;
+  p.wide = 0;
+  return p;
+}
 
 // A single pass of more (request, KV head, row tile) units than CUs runs
 // its eight-wave workgroups (one per CU) in rounds.  Two requests per
@@ -1618,6 +2097,8 @@ SplitPlan split_plan(const bc_shape& s, int nodes, int cus) {
     return parts < 2 ? p : SplitPlan{parts, tiles, waves};
   };
   const long long u = units > 0 ? units : 1;
+  const SplitPlan wide = wide_plan(s, row_tiles, max_tiles, cus);
+  if (wide.wide) return wide;
   // A single pass whose eight waves take two tiles or fewer each beats a
   // split, which adds the merge launch (one request over 256 tokens: 8.2
   // against 9.6 us, over 384: 8.4 against 9.3 us; 2 x 256: 8.5 against
@@ -1643,7 +2124,7 @@ SplitPlan split_plan(const bc_shape& s, int nodes, int cus) {
   return pair_requests(s.batch, u, eight, cus);
 }
 
-// Workspace of tree_split_kernel: P.parts (acc; max, sum) slots per output row.
+// Workspace of a split plan: P.parts (acc; max, sum) slots per output row.
 size_t split_workspace(const bc_shape& s, int nodes, const SplitPlan& plan, size_t* acc_bytes) {
   if (plan.parts < 2) return 0;
   const size_t slots = (size_t)s.batch * nodes * s.query_heads * plan.parts;
@@ -1662,6 +2143,12 @@ void launch_split_kernel(const TreeParams& P, const SplitPlan& plan, dim3 grid,
     tree_split_kernel<D, 8, 1><<<grid, 512, 0, st>>>(P);
 }
 
+template <int D>
+void launch_wide_kernel(const TreeParams& P, const SplitPlan& plan, dim3 grid, hipStream_t st) {
+  if (plan.wide == 2) tree_wide_kernel<D, 2><<<grid, 256, 0, st>>>(P);
+  else tree_wide_kernel<D, 4><<<grid, 256, 0, st>>>(P);
+}
+
 hipError_t launch_split(TreeParams& P, int dim, const SplitPlan& plan, void* workspace,
                         size_t acc_bytes, hipStream_t st) {
   P.parts = plan.parts;
@@ -1670,13 +2157,21 @@ hipError_t launch_split(TreeParams& P, int dim, const SplitPlan& plan, void* wor
     P.part_acc = static_cast<float*>(workspace);
     P.part_ml = reinterpret_cast<float*>(static_cast<char*>(workspace) + acc_bytes);
   }
-  const size_t groups = ((size_t)P.batch + plan.rq - 1) / plan.rq;
-  P.grid3d = groups <= 65535;
-  const dim3 grid = P.grid3d
-      ? dim3((unsigned)(P.hkv * P.row_tiles), (unsigned)groups, (unsigned)plan.parts)
-      : dim3((unsigned)((size_t)plan.parts * groups * P.hkv * P.row_tiles));
-  if (dim == 64) launch_split_kernel<64>(P, plan, grid, st);
-  else launch_split_kernel<128>(P, plan, grid, st);
+  if (plan.wide) {
+    const size_t groups =
+        (size_t)P.batch * P.hkv * ((P.row_tiles + plan.wide - 1) / plan.wide);
+    const dim3 grid((unsigned)(groups * plan.parts));
+    if (dim == 64) launch_wide_kernel<64>(P, plan, grid, st);
+    else launch_wide_kernel<128>(P, plan, grid, st);
+  } else {
+    const size_t groups = ((size_t)P.batch + plan.rq - 1) / plan.rq;
+    P.grid3d = groups <= 65535;
+    const dim3 grid = P.grid3d
+        ? dim3((unsigned)(P.hkv * P.row_tiles), (unsigned)groups, (unsigned)plan.parts)
+        : dim3((unsigned)((size_t)plan.parts * groups * P.hkv * P.row_tiles));
+    if (dim == 64) launch_split_kernel<64>(P, plan, grid, st);
+    else launch_split_kernel<128>(P, plan, grid, st);
+  }
   hipError_t err = hipGetLastError();
   if (err != hipSuccess || plan.parts < 2) return err;
   const size_t rows = (size_t)P.batch * P.nodes * P.hq;
@@ -1686,84 +2181,51 @@ hipError_t launch_split(TreeParams& P, int dim, const SplitPlan& plan, void* wor
   return hipGetLastError();
 }
 
+// One call, with the caller's workspace where it serves, else a slot of the
+// library's scratch pool, else (under graph capture, or for a plan larger
+// than a slot) without one.
+int tree_call(bc_shape s, bc_tree_inputs in, int nodes, void* workspace, size_t workspace_bytes,
+              bc_stream_t stream) {
+  if (!tree_args_ok(s, in, nodes)) return BC_ERROR_INVALID_VALUE;
+  TreeParams P = make_params(s, in, nodes);
+  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (!tree_ptrs_aligned(in) || !pool_known(s)) return launch_tree(P, s.dim, pool_known(s), st);
+  const int cus = bch::device_cus();
+  const bool ws_ok = workspace && aligned16(workspace);
+  size_t acc = 0;
+  const SplitPlan plan = split_plan(s, nodes, cus);
+  const size_t need = split_workspace(s, nodes, plan, &acc);
+  if (need == 0) return launch_split(P, s.dim, plan, nullptr, 0, st);
+  if (ws_ok && workspace_bytes >= need) return launch_split(P, s.dim, plan, workspace, acc, st);
+  const bch::ScratchLease lease(st, need);
+  if (lease.get()) return launch_split(P, s.dim, plan, lease.get(), acc, st);
+  // One part per unit.
+  const int max_tiles =
+      (s.max_pages * BC_PAGE_SIZE + kTile - 1) / kTile + (nodes + kTile - 1) / kTile;
+  SplitPlan one{1, (max_tiles + 1) / 2 * 2, 8};
+  one.wide = plan.wide;
+  if (!one.wide)
+    one = pair_requests(P.batch, (long long)P.batch * P.hkv * P.row_tiles, one, cus);
+  return launch_split(P, s.dim, one, nullptr, 0, st);
+}
+
 }  // namespace
 
 extern "C" int bc_tree_verify(bc_shape s, bc_tree_inputs in, int nodes,
                               bc_stream_t stream) {
-  if (!tree_args_ok(s, in, nodes)) return BC_ERROR_INVALID_VALUE;
-  TreeParams P = make_params(s, in, nodes);
-  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const bool vec = tree_ptrs_aligned(in);
-  const int cus = bch::device_cus();
-  const bool known = pool_known(s);
-  if (vec && known && !rows_kernel_for(P.batch, P.hkv, P.row_tiles, cus)) {
-    // The reference's signature has no workspace: a plan that splits the
-    // prefix borrows a slot of the library's scratch pool for the call
-    // (none under graph capture or when the slot is too small: the single
-    // pass below then runs).
-    const SplitPlan plan = split_plan(s, nodes, cus);
-    size_t acc = 0;
-    const size_t need = split_workspace(s, nodes, plan, &acc);
-    if (need > 0) {
-      const bch::ScratchLease lease(st, need);
-      if (lease.get()) return launch_split(P, s.dim, plan, lease.get(), acc, st);
-    }
-    const int max_tiles =
-        (s.max_pages * BC_PAGE_SIZE + kTile - 1) / kTile + (nodes + kTile - 1) / kTile;
-    const long long units = (long long)P.batch * P.hkv * P.row_tiles;
-    return launch_split(P, s.dim, pair_requests(P.batch, units, SplitPlan{1, max_tiles, 8}, cus),
-                        nullptr, 0, st);
-  }
-  return launch_tree(P, s.dim, vec, known, st);
+  return tree_call(s, in, nodes, nullptr, 0, stream);
 }
 
-namespace {
-
-bool tree_shape_ok(const bc_shape& s, int nodes) {
-  return s.batch >= 1 && s.query_heads >= 1 && s.kv_heads >= 1 &&
-         s.query_heads % s.kv_heads == 0 && (s.dim == 64 || s.dim == 128) &&
-         s.max_pages >= 1 && nodes >= 1 && nodes <= BC_MAX_TREE_NODES;
-}
-
-bool split_for(const bc_shape& s, int nodes) {
-  const int row_tiles = (nodes * (s.query_heads / s.kv_heads) + 31) / 32;
-  return !rows_kernel_for(s.batch, s.kv_heads, row_tiles, bch::device_cus());
-}
-
-// tree_rows_kernel, split plans of one part and calls without the pool size
-// need no workspace.
-size_t ws_size(const bc_shape& s, int nodes) {
-  if (!pool_known(s) || !split_for(s, nodes)) return 0;
-  size_t a = 0;
-  return split_workspace(s, nodes, split_plan(s, nodes, bch::device_cus()), &a);
-}
-
-int tree_ws_call(bc_shape s, bc_tree_inputs in, int nodes, void* workspace,
-                 size_t workspace_bytes, bc_stream_t stream) {
-  if (!tree_args_ok(s, in, nodes)) return BC_ERROR_INVALID_VALUE;
-  const bool vec = tree_ptrs_aligned(in);
-  // Tensors that are not 16-byte aligned, and calls without the pool size,
-  // take the single pass.
-  if (!vec || !pool_known(s)) return bc_tree_verify(s, in, nodes, stream);
-  if (!split_for(s, nodes)) return bc_tree_verify(s, in, nodes, stream);
-  const SplitPlan plan = split_plan(s, nodes, bch::device_cus());
-  size_t acc = 0;
-  const size_t need = split_workspace(s, nodes, plan, &acc);
-  if (!workspace || need == 0 || workspace_bytes < need || !aligned16(workspace))
-    return bc_tree_verify(s, in, nodes, stream);
-  TreeParams P = make_params(s, in, nodes);
-  return launch_split(P, s.dim, plan, workspace, acc, reinterpret_cast<hipStream_t>(stream));
-}
-
-}  // namespace
-
+// Calls without the pool size, and plans of one part, need no workspace.
 extern "C" size_t bc_tree_verify_workspace_size(bc_shape s, int nodes) {
-  if (!tree_shape_ok(s, nodes)) return 0;
-  return ws_size(s, nodes);
+  if (!tree_shape_ok(s, nodes) || !pool_known(s)) return 0;
+  const int cus = bch::device_cus();
+  size_t a = 0;
+  return split_workspace(s, nodes, split_plan(s, nodes, cus), &a);
 }
 
 extern "C" int bc_tree_verify_ws(bc_shape s, bc_tree_inputs in, int nodes,
                                  void* workspace, size_t workspace_bytes,
                                  bc_stream_t stream) {
-  return tree_ws_call(s, in, nodes, workspace, workspace_bytes, stream);
+  return tree_call(s, in, nodes, workspace, workspace_bytes, stream);
 }

@@ -1,0 +1,144 @@
+"""Tree verification of wide trees, at the edges of their tiles, steps and
+parts, against the CPU oracle.
+
+tree_wide_kernel shares K/V tiles between row tiles: two or four a workgroup,
+whole or in parts.  A call's shape decides; short lengths under large page
+tables keep the oracle cheap and leave parts empty.  The gate is the reference
+driver's 3e-4 (src/main.cu:505-509).
+"""
+
+import numpy as np
+import pytest
+import torch
+
+import branchcraft_capi as capi
+import gpu_helpers as G
+from oracle import oracle_np
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [0, 1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 127, 129, 200]
+
+
+def _case(seed, batch, nodes, hq, hkv, d, max_pages, pool=None, longest=0, parents="random"):
+    """Lengths from EDGES in a shuffled order (the first `longest` tokens, if
+    given), distinct pages, some of them outside the pool or with NaN past the
+    length."""
+    rng = np.random.default_rng(seed)
+    lengths = np.array([EDGES[i % len(EDGES)] for i in range(batch)], dtype=np.int32)
+    rng.shuffle(lengths)
+    lengths[0] = max(lengths[0], min(longest, max_pages * 16))
+    npg = [-(-int(x) // 16) for x in lengths]
+    used = sum(npg) + 1
+    pool = max(pool or 0, used)
+    ids = rng.permutation(pool).astype(np.int32)
+    # Only the pages in use are filled; the rest of a large pool stays zero.
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    k, v = (torch.zeros((pool, 16, hkv, d), device="cuda", dtype=torch.float16) for _ in range(2))
+    live = torch.from_numpy(ids[:used].astype(np.int64)).cuda()
+    for t in (k, v):
+        t[live] = torch.randn((used, 16, hkv, d), generator=g, device="cuda", dtype=torch.float16)
+    pages = np.full((batch, max_pages), -1, dtype=np.int32)
+    at = 0
+    for b in range(batch):
+        pages[b, :npg[b]] = ids[at:at + npg[b]]
+        at += npg[b]
+        if lengths[b] % 16:
+            last = int(pages[b, npg[b] - 1])
+            k[last, lengths[b] % 16:] = float("nan")
+            v[last, lengths[b] % 16:] = float("inf")
+    par = oracle_np.random_parents(rng, batch, nodes)
+    if parents == "chain":
+        par[:] = np.arange(-1, nodes - 1)
+    elif parents == "malformed":  # cycles, self-loops, parents out of range
+        par[1 % batch] = (np.arange(nodes) + 1) % nodes
+        par[2 % batch] = np.arange(nodes)
+        par[3 % batch, nodes // 2:] = nodes + 5
+        par[4 % batch, 1:] = -9
+    dq, dk, dv = (rng.standard_normal((batch, nodes, h, d)).astype(np.float16)
+                  for h in (hq, hkv, hkv))
+    return k, v, pages, lengths, dq, dk, dv, par.astype(np.int32)
+
+
+def _run(fix, workspace):
+    k, v, pages, lengths, dq, dk, dv, par = fix
+    b, n, hq, d = dq.shape
+    shape = capi.Shape(b, hq, k.shape[2], d, pages.shape[1], k.shape[0])
+    tp, tl, tq, tdk, tdv, tpar = (G.dev(x) for x in (pages, lengths, dq, dk, dv, par))
+    out = G.nan_out((b, n, hq, d), 0)
+    prefix = capi.Inputs(None, k.data_ptr(), v.data_ptr(), tp.data_ptr(), tl.data_ptr(), None)
+    ins = capi.TreeInputs(prefix, tq.data_ptr(), tdk.data_ptr(), tdv.data_ptr(),
+                          tpar.data_ptr(), out.data_ptr())
+    L = G.lib()
+    if workspace:
+        nbytes = L.bc_tree_verify_workspace_size(shape, n)
+        ws = torch.full((max(1, nbytes),), 0xff, device="cuda", dtype=torch.uint8)  # NaN partials
+        G.check(L.bc_tree_verify_ws(shape, ins, n, ws.data_ptr(), nbytes, G.stream()), "ws call")
+    else:
+        G.check(L.bc_tree_verify(shape, ins, n, G.stream()), "call")
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+def _check(fix, oracle, splits):
+    k, v, pages, lengths, dq, dk, dv, par = fix
+    b, n, hq, d = dq.shape
+    shape = capi.Shape(b, hq, k.shape[2], d, pages.shape[1], k.shape[0])
+    assert (G.lib().bc_tree_verify_workspace_size(shape, n) > 0) == splits
+    # The oracle sees the pages in use only, renumbered.
+    live = np.unique(pages[pages >= 0])
+    small = np.searchsorted(live, np.maximum(pages, live[0] if len(live) else 0)).astype(np.int32)
+    small[pages < 0] = -1
+    pick = torch.from_numpy(live.astype(np.int64)).cuda()
+    expected = oracle.tree(k[pick].cpu().numpy(), v[pick].cpu().numpy(), small, lengths, dq, dk,
+                           dv, par, threads=16)
+    for workspace in (True, False):
+        G.gate(_run(fix, workspace), expected, 3e-4, f"workspace={workspace}")
+
+
+@pytest.mark.parametrize("batch,nodes,hq,hkv,d,max_pages,splits,parents", [
+    (28, 24, 32, 8, 128, 14, False, "random"),    # three row tiles: an idle wave
+    (28, 32, 32, 8, 128, 14, False, "malformed"),  # four, exactly full
+    (28, 33, 32, 8, 128, 14, False, "chain"),     # five: a group of one; two draft tiles
+    (32, 100, 28, 4, 64, 14, False, "random"),    # group 7: 22 row tiles, partly filled rows
+    (7, 256, 32, 8, 128, 14, False, "chain"),     # the widest tree: eight draft tiles
+    (2, 256, 64, 8, 64, 14, False, "malformed"),
+    (64, 9, 32, 8, 64, 14, False, "random"),      # two row tiles, two workgroups per CU
+    (32, 16, 32, 8, 128, 60, False, "malformed"),  # two, one workgroup per CU
+    (20, 16, 32, 8, 128, 130, True, "random"),    # three parts
+    (32, 16, 32, 8, 128, 130, True, "chain"),     # two parts
+    (32, 64, 16, 16, 64, 130, False, "random"),   # D = 64: 512 groups, whole
+    (16, 64, 16, 16, 64, 130, True, "random"),    # D = 64: two parts
+])
+def test_wide_trees(batch, nodes, hq, hkv, d, max_pages, splits, parents, oracle):
+    fix = _case(batch + nodes, batch, nodes, hq, hkv, d, max_pages, parents=parents,
+                longest=1500 if max_pages > 100 else 0)
+    _check(fix, oracle, splits)
+
+
+def test_pages_outside_the_pool_are_skipped(oracle):
+    """Ids past the pool and negative ones inside a length: the result is the one
+    without those pages' tokens."""
+    for shape in ((28, 32, 32, 8, 128, 14, None),):
+        batch, nodes, hq, hkv, d, max_pages, pool = shape
+        k, v, pages, lengths, dq, dk, dv, par = _case(5, batch, nodes, hq, hkv, d, max_pages,
+                                                      pool=pool)
+        full = [b for b in range(batch) if lengths[b] >= 64]
+        bad = pages.copy()
+        cut, cut_len = np.full_like(pages, -1), lengths.copy()
+        for b in range(batch):
+            row = list(pages[b, :-(-int(lengths[b]) // 16)])
+            if b in full:
+                bad[b, 1] = k.shape[0] + 3 if b % 2 else -1
+                del row[1]
+                cut_len[b] -= 16
+            cut[b, :len(row)] = row
+        live = torch.from_numpy(np.unique(cut[cut >= 0]).astype(np.int64)).cuda()
+        ren = np.full(k.shape[0], -1, dtype=np.int32)
+        ren[live.cpu().numpy()] = np.arange(len(live))
+        small = np.where(cut >= 0, ren[np.maximum(cut, 0)], -1).astype(np.int32)
+        expected = oracle.tree(k[live].cpu().numpy(), v[live].cpu().numpy(), small, cut_len, dq,
+                               dk, dv, par, threads=16)
+        for workspace in (True, False):
+            got = _run((k, v, bad, lengths, dq, dk, dv, par), workspace)
+            G.gate(got, expected, 3e-4, f"{shape} workspace={workspace}")
