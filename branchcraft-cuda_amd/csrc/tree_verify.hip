@@ -32,6 +32,9 @@
 //  - tree_wide_kernel: trees of several row tiles per (request, KV head): four
 //    waves take four row tiles (or two, two waves each) and share K/V tiles
 //    that are loaded straight into LDS, whole prefixes or parts of them.
+//  - tree_flat_kernel: small trees over batches of long prefixes that stream
+//    from HBM: every workgroup takes an equal range of the batch's tiles, and
+//    merge_flat_kernel combines the units that a range boundary cuts.
 //  - tree_rows_kernel, tree_kernel: element-wise loads and stores, for tensors
 //    that are not 16-byte aligned (and, tree_kernel, calls without the pool
 //    size): a K/V tile shared by four row tiles, and one row tile each.
@@ -1187,7 +1190,7 @@ void launch_merge_split(const TreeParams& P, dim3 grid, hipStream_t st) {
   else merge_split_kernel<D, 4><<<grid, 256, 0, st>>>(P);
 }
 
-// ---- softmax pieces of tree_wide_kernel ----
+// ---- softmax pieces of tree_wide_kernel and tree_flat_kernel ----
 
 // Scores of the lane's query row at the tokens outside ok to -inf: sc[j] holds
 // token row 8*(j/4) + 4*g + j%4.
@@ -1642,6 +1645,539 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
                       acc[dt][4 * jq + 2] * inv, acc[dt][4 * jq + 3] * inv);
 }
 
+// ---- flat ranges: equal shares of a ragged batch's tiles ----
+
+// Tiles of one (KV head, row tile) of a request of length len: its draft
+// tiles, then its prefix tiles.
+__device__ __forceinline__ int flat_tiles(const TreeParams& P, int len) {
+  return (P.nodes + kTile - 1) / kTile + (len + kTile - 1) / kTile;
+}
+
+__device__ __forceinline__ int flat_len(const TreeParams& P, int b) {
+  return max(0, min(P.lengths[b], P.max_pages * BC_PAGE_SIZE));
+}
+
+__device__ __forceinline__ int wave_incl_scan_i(int x, int lane) {
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int y = __shfl_up(x, off, 64);
+    if (lane >= off) x += y;
+  }
+  return x;
+}
+
+// Lengths of 64 consecutive requests, lane i holding request base + i's, so
+// that stepping into the next request reads a register; a step out of the
+// window loads the one it needs.
+struct FlatLens {
+  int base, len;
+  __device__ __forceinline__ int at(const TreeParams& P, int lane, int b) {
+    if (b < base || b - base >= 64) {
+      base = b & ~63;
+      len = flat_len(P, min(base + lane, P.batch - 1));
+    }
+    return __builtin_amdgcn_readlane(len, __builtin_amdgcn_readfirstlane(b - base));
+  }
+};
+
+// Position in a range's tiles: tile t of segment `ord`, the part of unit
+// (z, b) that the range covers, which ends before tile tend; `rest` tiles of
+// the range follow the segment.
+struct FlatPos {
+  int ord, z, b, len, t, tend, rest;
+};
+
+// Range rid's first position (ord -1: the range is empty), of P.parts equal
+// ranges.  Units are ordered z (KV head, row tile) outermost, then request:
+// a range of one KV head's tiles finds requests that share pages next to
+// each other.
+__device__ __forceinline__ FlatPos flat_first(const TreeParams& P, int lane, int rid, int zdim,
+                                              FlatLens& lens) {
+  const int len0 = flat_len(P, min(lane, P.batch - 1));
+  int s = lane < P.batch ? flat_tiles(P, len0) : 0;
+  for (int base = 64; base < P.batch; base += 64) {
+    const int i = base + lane;
+    s += i < P.batch ? flat_tiles(P, flat_len(P, min(i, P.batch - 1))) : 0;
+  }
+  // The sum is the same in every lane; in a scalar register it keeps the
+  // whole walk scalar.
+  const int all = __builtin_amdgcn_readfirstlane(wave_sum_i(s));
+  const int total = all * zdim;
+  const int per = (total + P.parts - 1) / P.parts;
+  const int f0 = rid * per;
+  const int count = min(total - f0, per);
+  FlatPos p{-1, 0, 0, 0, 0, 0, 0};
+  lens = FlatLens{0, len0};
+  if (count <= 0) return p;
+  p.ord = 0;
+  p.z = f0 / all;
+  int rem = f0 - p.z * all;
+  for (int base = 0;; base += 64) {
+    if (base > 0) lens = FlatLens{base, flat_len(P, min(base + lane, P.batch - 1))};
+    const int n = base + lane < P.batch ? flat_tiles(P, lens.len) : 0;
+    const int inc = wave_incl_scan_i(n, lane);
+    const int tot = __builtin_amdgcn_readlane(inc, 63);
+    if (rem < tot) {
+      const unsigned long long hit = __builtin_amdgcn_ballot_w64(inc > rem);
+      const int first = __builtin_ffsll((long long)hit) - 1;
+      p.b = base + first;
+      p.t = rem - __builtin_amdgcn_readlane(inc - n, first);
+      p.len = __builtin_amdgcn_readlane(lens.len, first);
+      break;
+    }
+    rem -= tot;
+  }
+  p.tend = min(flat_tiles(P, p.len), p.t + count);
+  p.rest = count - (p.tend - p.t);
+  return p;
+}
+
+// The segment after p's (p.rest > 0): the next request, or the first one of
+// the next z.
+__device__ __forceinline__ void flat_next(const TreeParams& P, int lane, FlatLens& lens,
+                                          FlatPos& p) {
+  ++p.ord;
+  if (++p.b == P.batch) {
+    p.b = 0;
+    ++p.z;
+  }
+  p.len = lens.at(P, lane, p.b);
+  p.t = 0;
+  p.tend = min(flat_tiles(P, p.len), p.rest);
+  p.rest -= p.tend;
+}
+
+// Workgroup ids go round the eight XCDs: each XCD takes a contiguous eighth
+// of the ranges, so neighbouring ranges share an L2.
+__device__ __forceinline__ int flat_range_id(const TreeParams& P) {
+  const int n = P.parts, i = blockIdx.x;
+  return n % 8 == 0 ? i % 8 * (n / 8) + i / 8 : i;
+}
+
+// What merge_flat_kernel needs of each range, after the partials' (max, sum)
+// pairs (two slots of 32 rows per range): the unit it begins in and how many
+// tiles into it (an empty range: unit -1, tile 0).
+__device__ __forceinline__ int2* flat_records(const TreeParams& P) {
+  return reinterpret_cast<int2*>(P.part_ml + (size_t)P.parts * 2 * 32 * 2);
+}
+
+__device__ __forceinline__ void flat_record(const TreeParams& P, int rid, const FlatPos& p) {
+  if (threadIdx.x == 0)
+    flat_records(P)[rid] = p.ord < 0 ? make_int2(-1, 0) : make_int2(p.z * P.batch + p.b, p.t);
+}
+
+// Tree verification of a ragged batch in equal shares.  The batch's tiles
+// (per unit, a (KV head, row tile) of a request: its draft tiles, then its
+// prefix tiles) form one sequence, and workgroup r takes the r-th of
+// P.parts equal ranges of it, crossing unit boundaries as it goes: however
+// ragged the prefixes are, every workgroup streams the same number of
+// tiles.  Within a unit's segment the W waves take tiles round-robin, each
+// with its own staging area and no barrier; at the segment's end they merge
+// through LDS.  A unit that lies inside one range is written directly; the
+// others leave one FP32 partial per range (slot 2r for the range's first
+// segment, 2r + 1 for its last), which merge_flat_kernel combines.
+// Bound by HBM: a wave requests its next tile, also across a segment's end,
+// before it computes the current one, with non-temporal loads (plain ones: 13
+// us more at the shape below), ahead of the waves that compute.  64 requests x
+// 128-4096 tokens x 7 nodes (520 MB) take 126 us with a workgroup per two
+// requests, 100-105 us so (two boxes), 5 TB/s for the call.  Tile loads without
+// the math, reach 6.9 TB/s over prefixes of equal length; a ragged batch's
+// boundaries (partials, LDS merges, their kernel) cost 11 us, and four-wave
+// workgroups over 512 ranges would leave twice the partials (105 us).
+template <int D, int W>
+__global__ __launch_bounds__(64 * W, 2) void tree_flat_kernel(TreeParams P) {
+  constexpr int KS = D / 16;      // MFMA k-steps; also load instructions per tile
+  constexpr int DT = D / 32;      // 32-row output tiles over the head dimension
+  constexpr int KP = D + 8;       // halves per staged K row
+  constexpr int VP = D + 16;      // halves per staged V row
+  constexpr int LPR = D / 8;      // lanes per token row in a whole-row load
+  constexpr int RPI = 64 / LPR;   // token rows per load instruction
+  constexpr int LPP = KS / 2;     // load instructions per page
+  constexpr int STAGE = kTile * (KP + VP);  // halves per wave
+  constexpr int QPW = KS / W > 0 ? KS / W : 1;  // Q fragments loaded per wave
+
+  pin_params(P);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 5;   // lane half
+  const int lr = lane & 31;  // tile column (query row) / token slot
+
+  __shared__ __attribute__((aligned(16))) _Float16 s_stage[W * STAGE];
+  __shared__ uint4 s_q[KS * 64];            // Q^T fragments, lane-major per k-step
+  __shared__ int s_parent[BC_MAX_TREE_NODES];
+
+  const int rid = flat_range_id(P);
+  const int zdim = P.hkv * P.row_tiles;
+  const int ntd = (P.nodes + kTile - 1) / kTile;
+  FlatLens lens{0, 0};
+  FlatPos seg = flat_first(P, lane, rid, zdim, lens);
+  flat_record(P, rid, seg);
+  if (seg.ord < 0) return;  // uniform over the workgroup
+
+  // Page ids of a wave's tiles, every W-th from tile t of request b: lane i
+  // of a register holds page i % 2 of the i / 2-th of them, loaded from
+  // inside the request's table row.
+  constexpr int TPC = 32;  // tiles per register
+  auto load_ids = [&](int b, int t) {
+    const int pg = (t + W * (lane >> 1) - ntd) * (kTile / BC_PAGE_SIZE) + (lane & 1);
+    return P.pages[(size_t)b * P.max_pages + min(max(pg, 0), P.max_pages - 1)];
+  };
+
+  _Float16* const ks = s_stage + wave * STAGE;
+  _Float16* const vs = ks + kTile * KP;
+  const int trG = lane >> 4, trj = lane & 15;
+  const _Float16* vtr = vs + (4 * (trG >> 1) + (trj >> 2)) * VP + 16 * (trG & 1) + 4 * (trj & 3);
+  // Whole-row load geometry: load s of a lane covers token row
+  // s*RPI + lane/LPR, dims 8*(lane%LPR) .. +8.
+  const int lrow = lane / LPR, lcol = 8 * (lane % LPR);
+  const size_t tok_stride = (size_t)P.hkv * D;
+  unsigned loff[LPP];
+#pragma unroll
+  for (int j = 0; j < LPP; ++j)
+    loff[j] = (unsigned)((((size_t)(j * RPI + lrow)) * tok_stride + lcol) * sizeof(uint16_t));
+  const unsigned page_bytes = (unsigned)(BC_PAGE_SIZE * tok_stride * sizeof(uint16_t));
+
+  uint4 kreg[KS], vreg[KS];
+  // Tile t of unit (kvh, b) from page ids id0 and id1 (a draft tile's are
+  // unused).  Pages outside the pool read page 0, rows past the length their
+  // page's rows and draft rows past the node count the last node's: all in
+  // bounds, all masked.
+  auto issue = [&](int kvh, int b, int t, int id0, int id1) {
+    if (t >= ntd) {
+      const char* kb = reinterpret_cast<const char*>(P.k + (size_t)kvh * D);
+      const char* vb = reinterpret_cast<const char*>(P.v + (size_t)kvh * D);
+      unsigned long long off[2];
+      off[0] = (unsigned long long)((unsigned)id0 < (unsigned)P.phys_pages ? id0 : 0) * page_bytes;
+      off[1] = (unsigned long long)((unsigned)id1 < (unsigned)P.phys_pages ? id1 : 0) * page_bytes;
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+        kreg[s] = ldg16_stream(reinterpret_cast<const uint16_t*>(kb + off[s / LPP] + loff[s % LPP]));
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+        vreg[s] = ldg16_stream(reinterpret_cast<const uint16_t*>(vb + off[s / LPP] + loff[s % LPP]));
+    } else {
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const int dn = min(t * kTile + s * RPI + lrow, P.nodes - 1);
+        const size_t off = (((size_t)b * P.nodes + dn) * P.hkv + kvh) * D + lcol;
+        kreg[s] = ldg16(P.dk + off);
+        vreg[s] = ldg16(P.dv + off);
+      }
+    }
+  };
+  // Valid tokens of a tile (draft tiles: of the node count).
+  auto rows_of = [&](int len, int t, int id0, int id1) {
+    if (t >= ntd && (t + 1 - ntd) * kTile <= len && (unsigned)id0 < (unsigned)P.phys_pages &&
+        (unsigned)id1 < (unsigned)P.phys_pages)
+      return ~0u;
+    return (uint32_t)__builtin_amdgcn_readfirstlane(
+        t < ntd ? prefix_bits(P.nodes - t * kTile, 0, 0, 1)
+                : prefix_bits(len - (t - ntd) * kTile, id0, id1, P.phys_pages));
+  };
+
+  // ---- a segment's Q^T fragments and parents: registers, then LDS ----
+  uint4 qown[QPW];
+  int par_own = 0;
+  auto load_q = [&](int z, int b) {
+    const int kvh = div_by(z, P.row_tiles, P.rt_mul);
+    const int r = (z - kvh * P.row_tiles) * 32 + lr;
+    const int rnode = div_by(r, P.group, P.group_mul);
+    // Lanes past the tile's query rows read row (node 0, head 0), whose
+    // columns are never written out.
+    const int node = r < P.rows ? rnode : 0;
+    const int h = kvh * P.group + (r < P.rows ? r - rnode * P.group : 0);
+    const uint16_t* qp = P.dq + (((size_t)b * P.nodes + node) * P.hq + h) * D + 8 * g;
+#pragma unroll
+    for (int j = 0; j < QPW; ++j) qown[j] = ldg16(qp + 16 * min(wave + W * j, KS - 1));
+    par_own = P.parent[(size_t)b * P.nodes + min((int)threadIdx.x, P.nodes - 1)];
+  };
+  auto publish_q = [&]() {
+#pragma unroll
+    for (int j = 0; j < QPW; ++j)
+      if (wave + W * j < KS) s_q[(wave + W * j) * 64 + lane] = qown[j];
+    if ((int)threadIdx.x < P.nodes) s_parent[threadIdx.x] = par_own;
+  };
+  static_assert(BC_MAX_TREE_NODES <= 64 * W, "one parent entry per thread");
+
+  // Entering a segment: ids holds the page ids of this wave's first TPC
+  // tiles, ids_next the following ones and ids_seg the next segment's first.
+  int ids = load_ids(seg.b, seg.t + wave);
+  load_q(seg.z, seg.b);
+  FlatPos nseg = seg;
+  if (seg.rest > 0) flat_next(P, lane, lens, nseg);
+  int ids_next = load_ids(seg.b, seg.t + wave + W * TPC);
+  int ids_seg = load_ids(nseg.b, wave);
+  uint32_t rows = 0;     // valid tokens of the tile in the registers
+  bool loaded = false;   // whether it is the segment's first
+  publish_q();
+  __syncthreads();
+
+  f32x16 acc[DT];
+  for (;;) {
+    const int t0 = seg.t;
+    float m = kNegInf, l = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) acc[dt][j] = 0.f;
+    const int kvh = div_by(seg.z, P.row_tiles, P.rt_mul);
+    const int kvh_n = div_by(nseg.z, P.row_tiles, P.rt_mul);
+    const int rt = seg.z - kvh * P.row_tiles;
+    const int r = rt * 32 + lr;
+    const int node = r < P.rows ? div_by(r, P.group, P.group_mul) : 0;
+    // A round loads the wave's next tile -- of this segment, or the next
+    // one's first -- between staging its current one and the math on it.  A
+    // segment whose first tile is not in the registers yet begins with a
+    // round that only loads it.
+    for (int t = loaded ? t0 + wave : t0 + wave - W, i = loaded ? 0 : -1; t < seg.tend; t += W) {
+      const bool math = i >= 0;
+      const uint32_t now = rows;
+      // A wave about to load goes ahead of one that computes.
+      __builtin_amdgcn_s_setprio(2);
+      if (math) {
+        // Stage the tile; V rows that are not valid tokens may hold any bits
+        // (NaN included): their weight is zero, so the rows must be zero.
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          *reinterpret_cast<uint4*>(ks + (s * RPI + lrow) * KP + lcol) = kreg[s];
+          *reinterpret_cast<uint4*>(vs + (s * RPI + lrow) * VP + lcol) = vreg[s];
+        }
+        if (now != ~0u) {  // uniform
+#pragma unroll
+          for (int s = 0; s < KS; ++s)
+            if (!((now >> (s * RPI + lrow)) & 1u))
+              *reinterpret_cast<uint4*>(vs + (s * RPI + lrow) * VP + lcol) =
+                  make_uint4(0, 0, 0, 0);
+        }
+      }
+      wave_lds_sync();
+      const bool here = t + W < seg.tend;
+      loaded = !here && seg.rest > 0 && wave < nseg.tend;
+      if (here && ++i == TPC) {
+        i = 0;
+        ids = ids_next;
+        ids_next = load_ids(seg.b, t + W + W * TPC);
+      }
+      if (here || loaded) {
+        const int v = here ? ids : ids_seg, at = here ? 2 * i : 0, tn = here ? t + W : wave;
+        const int id0 = __builtin_amdgcn_readlane(v, at);
+        const int id1 = __builtin_amdgcn_readlane(v, at + 1);
+        issue(here ? kvh : kvh_n, here ? seg.b : nseg.b, tn, id0, id1);
+        rows = rows_of(here ? seg.len : nseg.len, tn, id0, id1);
+      }
+      __builtin_amdgcn_s_setprio(0);
+      if (!math) continue;
+      // ---- S^T = K Q^T ----
+      f32x16 sc[1];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) sc[0][j] = 0.f;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const uint4 k0 = *reinterpret_cast<const uint4*>(ks + lr * KP + 16 * s + 8 * g);
+        sc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16x8(k0), as_f16x8(s_q[s * 64 + lane]),
+                                                       sc[0], 0, 0, 0);
+      }
+      if (now != ~0u || t < ntd) {
+        uint32_t ok = now;
+        if (t < ntd) {  // the row's ancestor-or-self set
+          const int tbase = t * kTile;
+          ok = 0;
+          int cur = node;
+          for (int steps = 0; steps < P.nodes && cur >= 0 && cur < P.nodes; ++steps) {
+            if (cur >= tbase && cur < tbase + kTile) ok |= 1u << (cur - tbase);
+            cur = s_parent[cur];
+          }
+        }
+        row_mask(sc[0], ok, g);
+      }
+      row_max<DT, 1>(sc, P.scale_log2, m, l, acc);
+      const float mb = safe_max(m);
+      f16x8 pb[2], pl[2];
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) row_weights(sc[0], hh, P.scale_log2, mb, l, pb[hh], pl[hh]);
+      tile_pv<D, false>(vtr, pb, pl, acc);
+      wave_lds_sync();
+    }
+
+    // ---- segment end: merge the W waves through LDS, write, move on ----
+    const bool more = seg.rest > 0;
+    if (more) load_q(nseg.z, nseg.b);
+    l += shfl_xor_f(l, 32);  // both lane halves share m
+    constexpr int XP = D + 4;
+    constexpr int XW = STAGE / 2;  // floats in a wave's staging area
+    static_assert(32 * XP + 64 <= XW, "a wave's state fits its staging area");
+    auto xw = [&](int w) { return reinterpret_cast<float*>(s_stage) + (size_t)w * XW; };
+    {
+      float* dst = xw(wave) + (size_t)lr * XP;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int jq = 0; jq < 4; ++jq)
+          *reinterpret_cast<float4*>(dst + 32 * dt + 8 * jq + 4 * g) =
+              make_float4(acc[dt][4 * jq], acc[dt][4 * jq + 1], acc[dt][4 * jq + 2],
+                          acc[dt][4 * jq + 3]);
+      if (g == 0) *reinterpret_cast<float2*>(xw(wave) + 32 * XP + 2 * lr) = make_float2(m, l);
+    }
+    __syncthreads();
+    constexpr int TPR = 2 * W;    // threads per row
+    constexpr int DPT = D / TPR;  // dims per thread
+    static_assert(DPT % 4 == 0, "float4 steps");
+    const int mrow = threadIdx.x / TPR;
+    const int md0 = (threadIdx.x % TPR) * DPT;
+    const int rr = rt * 32 + mrow;
+    float mw[W], mm = kNegInf;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      mw[w] = xw(w)[32 * XP + 2 * mrow];
+      mm = __builtin_fmaxf(mm, mw[w]);
+    }
+    const float ms = safe_max(mm);
+    float ll = 0.f, o[DPT];
+#pragma unroll
+    for (int j = 0; j < DPT; ++j) o[j] = 0.f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float wt = fast_exp2(mw[w] - ms);  // 0 for a wave without tiles
+      ll += wt * xw(w)[32 * XP + 2 * mrow + 1];
+      const float* src = xw(w) + (size_t)mrow * XP + md0;
+#pragma unroll
+      for (int j = 0; j < DPT; j += 4) {
+        const float4 v4 = *reinterpret_cast<const float4*>(src + j);
+        o[j] += wt * v4.x;
+        o[j + 1] += wt * v4.y;
+        o[j + 2] += wt * v4.z;
+        o[j + 3] += wt * v4.w;
+      }
+    }
+    if (rr < P.rows) {
+      if (t0 == 0 && seg.tend == flat_tiles(P, seg.len)) {  // the whole unit
+        const int rrn = div_by(rr, P.group, P.group_mul);
+        const size_t orow = ((size_t)seg.b * P.nodes + rrn) * P.hq + kvh * P.group +
+                            (rr - rrn * P.group);
+        const float inv = 1.f / ll;  // every row sees its own node: ll > 0
+        float* dst = P.out + orow * D + md0;
+#pragma unroll
+        for (int j = 0; j < DPT; j += 4)
+          *reinterpret_cast<float4*>(dst + j) =
+              make_float4(o[j] * inv, o[j + 1] * inv, o[j + 2] * inv, o[j + 3] * inv);
+      } else {
+        const size_t slot = ((size_t)2 * rid + (seg.ord > 0)) * 32 + mrow;
+        float* dst = P.part_acc + slot * D + md0;
+#pragma unroll
+        for (int j = 0; j < DPT; j += 4)
+          *reinterpret_cast<float4*>(dst + j) = make_float4(o[j], o[j + 1], o[j + 2], o[j + 3]);
+        if (md0 == 0) *reinterpret_cast<float2*>(P.part_ml + 2 * slot) = make_float2(mm, ll);
+      }
+    }
+    if (!more) return;
+    publish_q();
+    seg = nseg;
+    ids = ids_seg;
+    if (seg.rest > 0) flat_next(P, lane, lens, nseg);
+    ids_next = load_ids(seg.b, wave + W * TPC);
+    ids_seg = load_ids(nseg.b, wave);
+    __syncthreads();
+  }
+}
+
+// Combines tree_flat_kernel's partials: one workgroup per range boundary r.
+// The unit that
+// range r starts inside is merged at the first boundary that cuts it, over
+// range r - 1 and the ranges from r on that start inside it too; every other
+// unit lies inside one range and was written by the attention kernel.  Range
+// r - 1 holds the unit as its first segment (slot 2(r - 1)) or, when the
+// unit begins inside it, its last (slot 2(r - 1) + 1); the others as their
+// first.
+template <int D>
+__global__ __launch_bounds__(256) void merge_flat_kernel(TreeParams P) {
+  pin_params(P);
+  constexpr int NF = D / 32;  // float4s per thread: 8 threads per row
+  constexpr int U = 4;        // parts loaded together
+  const int lane = threadIdx.x & 63;
+  const int r = 1 + blockIdx.x;
+  const int2* rec = flat_records(P);
+  const int2 m1 = rec[r], m0 = rec[r - 1];
+  const int mv = rec[min(r + 1 + lane, P.parts - 1)].x;
+  const int unit = m1.x;
+  if (m1.y == 0) return;                       // r starts on a unit's first tile
+  if (m0.x == unit && m0.y > 0) return;        // an earlier boundary cuts the unit too
+  // The ranges after r that start inside the unit follow r: count them.
+  int nparts = 2;
+  for (int base = r + 1;; base += 64) {
+    const int rr = base + lane;
+    const int x = base == r + 1 ? mv : rec[min(rr, P.parts - 1)].x;
+    const unsigned long long hit = __builtin_amdgcn_ballot_w64(rr < P.parts && x == unit);
+    const int n = ~hit ? __builtin_ffsll((long long)~hit) - 1 : 64;
+    nparts += n;
+    if (n < 64 || base + 64 >= P.parts) break;
+  }
+  const int row = threadIdx.x >> 3, d0 = 4 * (threadIdx.x & 7);
+  const int z = unit / P.batch, b = unit - z * P.batch;
+  const int kvh = div_by(z, P.row_tiles, P.rt_mul);
+  const int rr = (z - kvh * P.row_tiles) * 32 + row;
+  if (rr >= P.rows) return;
+  const int first = 2 * (r - 1) + (m0.x != unit);
+  auto slot_of = [&](int p) { return p == 0 ? first : 2 * (r - 1 + p); };
+  float mm = kNegInf, lsum = 0.f;
+  float4 a[NF];
+#pragma unroll
+  for (int j = 0; j < NF; ++j) a[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int p0 = 0; p0 < nparts; p0 += U) {
+    float2 ml[U];
+    float4 v[U][NF];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t at = (size_t)slot_of(min(p0 + u, nparts - 1)) * 32 + row;
+      ml[u] = *reinterpret_cast<const float2*>(P.part_ml + 2 * at);
+#pragma unroll
+      for (int j = 0; j < NF; ++j)
+        v[u][j] = *reinterpret_cast<const float4*>(P.part_acc + at * D + 32 * j + d0);
+    }
+    float mn = mm;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      mn = __builtin_fmaxf(mn, p0 + u < nparts ? ml[u].x : kNegInf);
+    const float ms = safe_max(mn);
+    const float a1 = fast_exp2(mm - ms);
+    lsum *= a1;
+#pragma unroll
+    for (int j = 0; j < NF; ++j) {
+      a[j].x *= a1;
+      a[j].y *= a1;
+      a[j].z *= a1;
+      a[j].w *= a1;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float w = p0 + u < nparts ? fast_exp2(ml[u].x - ms) : 0.f;
+      lsum += w * ml[u].y;
+#pragma unroll
+      for (int j = 0; j < NF; ++j) {
+        a[j].x += w * v[u][j].x;
+        a[j].y += w * v[u][j].y;
+        a[j].z += w * v[u][j].z;
+        a[j].w += w * v[u][j].w;
+      }
+    }
+    mm = mn;
+  }
+  const float inv = 1.f / lsum;  // every row sees its own node
+  const int rrn = div_by(rr, P.group, P.group_mul);
+  float* dst = P.out +
+               (((size_t)b * P.nodes + rrn) * P.hq + kvh * P.group + (rr - rrn * P.group)) * D + d0;
+#pragma unroll
+  for (int j = 0; j < NF; ++j)
+    *reinterpret_cast<float4*>(dst + 32 * j) =
+        make_float4(a[j].x * inv, a[j].y * inv, a[j].z * inv, a[j].w * inv);
+}
+
+// Wide trees: RT row tiles of a (request, KV head) per workgroup (four
+// waves, 4 / RT of them on each row tile), which share every K/V tile
+// through LDS.  A step is two 32-token tiles; with RT = 4 each wave takes
+// both, with RT = 2 one of them.  Steps form flat ranges as in
+// tree_flat_kernel.  Each step's loads are issued a step ahead into
+// registers and staged into the other LDS buffer after the step's math, one
+// barrier per step.
 // Row-sharing variant, for tensors that are not 16-byte aligned, of trees of
 // four or more row tiles per (request, KV head), where tree_kernel would read
 // the prefix once per row tile: the four
@@ -2181,6 +2717,52 @@ hipError_t launch_split(TreeParams& P, int dim, const SplitPlan& plan, void* wor
   return hipGetLastError();
 }
 
+// ---- tree_flat_kernel: ranges, workspace and launch ----
+
+// Ranges of tree_flat_kernel (0: not taken): one eight-wave workgroup per CU
+// for batches that stream their prefixes from HBM.  The lengths are on the
+// device, so the shape decides: small trees (one row tile), page tables of at
+// least 2048 tokens that could hold 400 MB, and a pool of at least 128 MB (a
+// smaller one stays in the 256 MB cache, where equal shares gain nothing:
+// requests that share their pages).  Same box, 7 nodes, tree_split_kernel
+// first: 64 x 128-4096 tokens 126 against 105 us, 24 x 128-4096 57 against 42,
+// 20 x 256-8192 87 against 62, 64 x 4096 equal lengths 195 against 190, 64 x
+// 128-4096 at D = 64 73 against 58; below the lines it loses: 64 x 32-1024
+// 32 against 44, 32 x 64-2048 28 against 38, 16 x 128-4096 28 against 33, 32 x
+// 2048 on shared pages 22 against 25 us.
+int flat_ranges(const bc_shape& s, int nodes, int cus) {
+  const int group = s.query_heads / s.kv_heads;
+  const long long page = 2LL * BC_PAGE_SIZE * s.kv_heads * s.dim * sizeof(uint16_t);
+  const long long table = (long long)s.batch * s.max_pages;  // pages
+  if ((long long)nodes * group > 32 || s.max_pages * BC_PAGE_SIZE < 2048 ||
+      table * page < 400000000LL || s.physical_pages * page < 128000000LL)
+    return 0;
+  if (table * s.kv_heads >= 1LL << 30) return 0;  // tile indices stay in an int
+  return cus;
+}
+
+size_t flat_workspace(const bc_shape& s, int ranges, size_t* acc_bytes) {
+  const size_t slots = (size_t)2 * ranges * 32;
+  *acc_bytes = slots * s.dim * sizeof(float);
+  return *acc_bytes + slots * 2 * sizeof(float) + (size_t)ranges * sizeof(int2);
+}
+
+template <int D>
+void launch_flat_kernel(const TreeParams& P, hipStream_t st) {
+  tree_flat_kernel<D, 8><<<dim3(P.parts), 512, 0, st>>>(P);
+  if (P.parts > 1) merge_flat_kernel<D><<<dim3(P.parts - 1), 256, 0, st>>>(P);
+}
+
+hipError_t launch_flat(TreeParams& P, int dim, int ranges, void* workspace, size_t acc_bytes,
+                       hipStream_t st) {
+  P.parts = ranges;
+  P.part_acc = static_cast<float*>(workspace);
+  P.part_ml = reinterpret_cast<float*>(static_cast<char*>(workspace) + acc_bytes);
+  if (dim == 64) launch_flat_kernel<64>(P, st);
+  else launch_flat_kernel<128>(P, st);
+  return hipGetLastError();
+}
+
 // One call, with the caller's workspace where it serves, else a slot of the
 // library's scratch pool, else (under graph capture, or for a plan larger
 // than a slot) without one.
@@ -2193,6 +2775,13 @@ int tree_call(bc_shape s, bc_tree_inputs in, int nodes, void* workspace, size_t 
   const int cus = bch::device_cus();
   const bool ws_ok = workspace && aligned16(workspace);
   size_t acc = 0;
+  if (const int flat = flat_ranges(s, nodes, cus)) {
+    const size_t need = flat_workspace(s, flat, &acc);
+    if (ws_ok && workspace_bytes >= need)
+      return launch_flat(P, s.dim, flat, workspace, acc, st);
+    const bch::ScratchLease lease(st, need);
+    if (lease.get()) return launch_flat(P, s.dim, flat, lease.get(), acc, st);
+  }
   const SplitPlan plan = split_plan(s, nodes, cus);
   const size_t need = split_workspace(s, nodes, plan, &acc);
   if (need == 0) return launch_split(P, s.dim, plan, nullptr, 0, st);
@@ -2221,6 +2810,7 @@ extern "C" size_t bc_tree_verify_workspace_size(bc_shape s, int nodes) {
   if (!tree_shape_ok(s, nodes) || !pool_known(s)) return 0;
   const int cus = bch::device_cus();
   size_t a = 0;
+  if (const int flat = flat_ranges(s, nodes, cus)) return flat_workspace(s, flat, &a);
   return split_workspace(s, nodes, split_plan(s, nodes, cus), &a);
 }
 

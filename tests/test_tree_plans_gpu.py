@@ -1,10 +1,12 @@
-"""Tree verification of wide trees, at the edges of their tiles, steps and
-parts, against the CPU oracle.
+"""Tree verification plans of batched and wide trees, at the edges of their
+tiles, steps, parts and ranges, against the CPU oracle.
 
 tree_wide_kernel shares K/V tiles between row tiles: two or four a workgroup,
-whole or in parts.  A call's shape decides; short lengths under large page
-tables keep the oracle cheap and leave parts empty.  The gate is the reference
-driver's 3e-4 (src/main.cu:505-509).
+whole or in parts.  tree_flat_kernel walks equal ranges of a ragged batch's
+tiles.  Which one a call takes follows from its shape, so each case's shape
+puts it on one of them; short lengths under large page tables keep the oracle
+cheap and leave parts and ranges empty.  The gate is the reference driver's
+3e-4 (src/main.cu:505-509).
 """
 
 import numpy as np
@@ -116,10 +118,24 @@ def test_wide_trees(batch, nodes, hq, hkv, d, max_pages, splits, parents, oracle
     _check(fix, oracle, splits)
 
 
+@pytest.mark.parametrize("batch,nodes,hq,hkv,d,max_pages,pool,longest,parents", [
+    (64, 7, 32, 8, 128, 128, 2048, 2048, "random"),
+    (50, 1, 32, 8, 128, 129, 2048, 0, "random"),     # one node: one-tile units
+    (64, 32, 8, 8, 128, 128, 2048, 700, "malformed"),  # a full draft tile
+    (130, 8, 8, 2, 128, 200, 8192, 3200, "random"),  # lengths in several windows of 64
+    (64, 31, 16, 16, 64, 128, 2048, 1000, "chain"),  # 31 draft tokens
+    (300, 4, 7, 1, 128, 200, 16384, 2000, "random"),  # more requests than ranges
+])
+def test_flat_ranges(batch, nodes, hq, hkv, d, max_pages, pool, longest, parents, oracle):
+    fix = _case(batch + nodes, batch, nodes, hq, hkv, d, max_pages, pool=pool, longest=longest,
+                parents=parents)
+    _check(fix, oracle, True)
+
+
 def test_pages_outside_the_pool_are_skipped(oracle):
-    """Ids past the pool and negative ones inside a length: the result is the one
-    without those pages' tokens."""
-    for shape in ((28, 32, 32, 8, 128, 14, None),):
+    """Ids past the pool and negative ones inside a length, on the wide and the
+    flat kernel: the result is the one without those pages' tokens."""
+    for shape in ((28, 32, 32, 8, 128, 14, None), (64, 7, 32, 8, 128, 128, 2048)):
         batch, nodes, hq, hkv, d, max_pages, pool = shape
         k, v, pages, lengths, dq, dk, dv, par = _case(5, batch, nodes, hq, hkv, d, max_pages,
                                                       pool=pool)
