@@ -15,6 +15,8 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cstdint>
+#include <vector>
 
 #include "branchcraft.h"
 
@@ -364,6 +366,26 @@ void write_prefix_hip(at::Tensor& cache_k, at::Tensor& cache_v, const at::Tensor
                "write_prefix_");
 }
 
+// A host list as an int32 tensor on `like`'s device, written in stream order
+// by kernels that carry the values as arguments.
+at::Tensor int_tensor_hip(const at::Tensor& like, at::IntArrayRef values) {
+  TORCH_CHECK(values.size() <= INT32_MAX, "int_tensor: too many values");
+  std::vector<int32_t> host(values.size());
+  for (size_t i = 0; i < values.size(); ++i) {
+    TORCH_CHECK(values[i] >= INT32_MIN && values[i] <= INT32_MAX,
+                "int_tensor: value out of range");
+    host[i] = int32_t(values[i]);
+  }
+  const c10::DeviceGuard guard(like.device());
+  auto out = at::empty({int64_t(host.size())},
+                       at::TensorOptions().dtype(at::kInt).device(like.device()));
+  if (!host.empty())
+    check_launch(bc_write_ints(out.data_ptr<int>(), host.data(), int(host.size()),
+                               current_stream()),
+                 "int_tensor");
+  return out;
+}
+
 }  // namespace
 
 TORCH_LIBRARY(branchcraft, m) {
@@ -373,6 +395,7 @@ TORCH_LIBRARY(branchcraft, m) {
   m.def("copy_pages_(Tensor(a!) cache_k, Tensor(b!) cache_v, Tensor src_pages, Tensor dst_pages) -> ()");
   m.def("commit_paths_(Tensor(a!) cache_k, Tensor(b!) cache_v, Tensor draft_k, Tensor draft_v, Tensor requests, Tensor path_nodes, Tensor dest_pages, Tensor dest_slots) -> ()");
   m.def("write_prefix_(Tensor(a!) cache_k, Tensor(b!) cache_v, Tensor k, Tensor v, int[] pages) -> ()");
+  m.def("int_tensor(Tensor like, int[] values) -> Tensor");
   m.def("paged_decode(Tensor q, Tensor k, Tensor v, Tensor pages, Tensor lengths, int splits=0) -> Tensor");
 }
 
@@ -383,5 +406,6 @@ TORCH_LIBRARY_IMPL(branchcraft, CUDA, m) {
   m.impl("copy_pages_", copy_pages_hip);
   m.impl("commit_paths_", commit_paths_hip);
   m.impl("write_prefix_", write_prefix_hip);
+  m.impl("int_tensor", int_tensor_hip);
   m.impl("paged_decode", paged_decode_hip);
 }

@@ -30,7 +30,7 @@ BC_MAX_TREE_NODES = 256
 EXPORTED = (
     "bc_decode", "bc_auto_splits", "bc_tree_verify",
     "bc_tree_verify_workspace_size", "bc_tree_verify_ws", "bc_commit_path", "bc_commit_paths", "bc_copy_pages",
-    "bc_write_prefix", "bc_packed_decode", "bc_packed_decode_workspace_size",
+    "bc_write_prefix", "bc_write_ints", "bc_packed_decode", "bc_packed_decode_workspace_size",
     "bc_packed_decode_ws", "bc_packed_decode_noalloc", "bc_version",
 )
 
@@ -91,6 +91,8 @@ def load(path: str | Path | None = None) -> ctypes.CDLL:
                                     c_longlong, c_longlong, c_void_p, c_void_p,
                                     POINTER(c_int32), c_int, c_void_p]
     lib.bc_write_prefix.restype = c_int
+    lib.bc_write_ints.argtypes = [c_void_p, POINTER(c_int32), c_int, c_void_p]
+    lib.bc_write_ints.restype = c_int
     lib.bc_packed_decode.argtypes = [Shape, c_void_p, c_void_p, c_void_p, c_void_p,
                                      c_void_p, c_longlong, c_longlong, c_longlong,
                                      c_longlong, c_float, c_void_p]

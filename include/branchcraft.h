@@ -239,6 +239,15 @@ int bc_write_prefix(bc_shape shape, const bc_half* k, const bc_half* v,
                     bc_half* cache_k, bc_half* cache_v,
                     const int32_t* host_pages, int tokens, bc_stream_t stream);
 
+/* dst[i] = host_values[i], i < count: a host list (a request's page table, the
+ * rows of a commit) into device memory, in stream order.  host_values is HOST
+ * memory, read before the call returns: the values travel in the kernel
+ * arguments, 896 per launch, so the host waits for nothing.  No reference
+ * counterpart: it replaces the index tensors of
+ * python/branchcraft_torch/transaction.py:94-148. */
+int bc_write_ints(int32_t* dst, const int32_t* host_values, int count,
+                  bc_stream_t stream);
+
 /* vLLM-style packed-cache decode with FP16 output.  Token t of sequence b
  * lives at element offset
  *   pages[b, t/16]*block_stride + kvh*head_stride + (t%16)*slot_stride
