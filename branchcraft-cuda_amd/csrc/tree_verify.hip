@@ -31,7 +31,8 @@
 //    pages run on the same XCD and reuse its L2.
 //  - tree_wide_kernel: trees of several row tiles per (request, KV head): four
 //    waves take four row tiles (or two, two waves each) and share K/V tiles
-//    that are loaded straight into LDS, whole prefixes or parts of them.
+//    that are loaded straight into LDS, whole units or shares of them, which
+//    merge_wide_kernel combines.
 //  - tree_flat_kernel: small trees over batches of long prefixes that stream
 //    from HBM: every workgroup takes an equal range of the batch's tiles, and
 //    merge_flat_kernel combines the units that a range boundary cuts.
@@ -77,7 +78,9 @@ struct TreeParams {
   int rows, row_tiles;      // rows = nodes * group per (request, KV head)
   float scale_log2;
   // tree_split_kernel: parts per unit and tiles per part; with parts > 1,
-  // part_acc/part_ml hold P.parts slots per output row.
+  // part_acc/part_ml hold P.parts slots per output row.  tree_wide_kernel:
+  // workgroups that split the units (1: none are split), with a slot per
+  // workgroup and row of its, and the CUs they run on.
   int parts, tiles_per_part;
   // ceil(2^32 / d) for d = group and d = row_tiles (0: divide plainly), and
   // whether the launch is a (KV head x row tile, request group, part) grid.
@@ -1271,21 +1274,135 @@ __device__ __forceinline__ void load_to_lds(const void* base, unsigned off, unsi
 
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// Tiles of one (KV head, row tile) of a request of length len: its draft
+// tiles, then its prefix tiles.
+__device__ __forceinline__ int flat_tiles(const TreeParams& P, int len) {
+  return (P.nodes + kTile - 1) / kTile + (len + kTile - 1) / kTile;
+}
+
+__device__ __forceinline__ int flat_len(const TreeParams& P, int b) {
+  return max(0, min(P.lengths[b], P.max_pages * BC_PAGE_SIZE));
+}
+
+// A workgroup's share of a wide tree: steps [t0, tend) of unit (request b, z =
+// (KV head, row group)), one of `parts` shares of the unit.
+struct WidePart {
+  int b, z, len, t0, tend, parts;
+};
+
+constexpr int kWideStep = 2 * kTile;     // tokens per step
+constexpr int kWideRequests = 4 * 64;    // requests of a split launch, four per lane
+constexpr int kWideParts = 63;           // most shares of a unit
+constexpr int kWideLeast = 6;            // fewest steps per share of a long unit
+constexpr float kWideSlack = 12.f;       // steps that a batch's partials cost
+
+// Per request: the first of its shares in the launch's order, and how many.
+// They stand after the partials' (max, sum) pairs.
+template <int RT>
+__device__ __forceinline__ int2* wide_records(const TreeParams& P) {
+  return reinterpret_cast<int2*>(P.part_ml + (size_t)P.parts * RT * 32 * 2);
+}
+
+// Workgroup blockIdx.x's share when P.parts workgroups split the units on
+// P.tiles_per_part CUs: the shortest share of at least kWideLeast steps with
+// which the batch, however ragged, needs no more than P.parts workgroups,
+// from the lengths themselves (parts == 0: none left).  A request's units
+// take equal shares.
+// Every wave finds it for itself, a lane holding four requests; counts of a
+// share per lane add up by ballots of their six bits.
+template <int RT>
+__device__ __forceinline__ WidePart wide_part(const TreeParams& P, int lane, int zdim) {
+  constexpr int NW = kWideRequests / 64;
+  int len[NW], steps[NW], sum = 0, most = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    len[w] = steps[w] = 0;
+    if (64 * w < P.batch) {  // uniform
+      len[w] = flat_len(P, min(64 * w + lane, P.batch - 1));
+      steps[w] = 64 * w + lane < P.batch ? (flat_tiles(P, len[w]) + 1) / 2 : 0;
+    }
+    sum += steps[w];
+    most = max(most, steps[w]);
+  }
+  // Uniform values in scalar registers keep the search scalar.
+  const int all = __builtin_amdgcn_readfirstlane(wave_sum_i(sum));
+  const int longest = __builtin_amdgcn_readfirstlane((int)wave_max((float)most));
+  const int cap = P.parts / zdim;  // shares of all requests, >= P.batch
+  // About ceil(steps / per): 1 to kWideParts, no more than steps, and 1 for
+  // per == longest.  Shares follow from the count, so that it need not be exact.
+  auto shares = [&](int w, int per) {
+    return max((int)((float)steps[w] * __builtin_amdgcn_rcpf((float)per) + 0.999f), min(steps[w], 1));
+  };
+  int per = max(max((all + cap - 1) / cap, (longest + kWideParts - 1) / kWideParts),
+                kWideLeast);
+  // An even batch (equal lengths, most CUs with a unit) gains nothing that
+  // its partials would not cost: whole units.
+  if ((float)longest <= (float)all * (float)zdim / (float)P.tiles_per_part + kWideSlack)
+    per = max(per, longest);
+  for (int hi = max(per, longest); per < hi;) {
+    const int mid = (per + hi) >> 1;
+    int total = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+      if (64 * w < P.batch) {
+        const int n = shares(w, mid);
+#pragma unroll
+        for (int bit = 0; bit < 6; ++bit)
+          total += __builtin_popcountll(__builtin_amdgcn_ballot_w64((n >> bit) & 1)) << bit;
+      }
+    if (total <= cap) hi = mid;
+    else per = mid + 1;
+  }
+  WidePart p{0, 0, 0, 0, 0, 0};
+  const int idx = blockIdx.x / zdim;
+  p.z = blockIdx.x - idx * zdim;
+  int before = 0;  // shares of the requests of earlier windows
+#pragma unroll
+  for (int w = 0; w < NW; ++w)
+    if (64 * w < P.batch) {
+      const int n = shares(w, per);
+      int pre = before, total = 0;
+#pragma unroll
+      for (int bit = 0; bit < 6; ++bit) {
+        const unsigned long long set = __builtin_amdgcn_ballot_w64((n >> bit) & 1);
+        pre += __builtin_amdgcn_mbcnt_hi((unsigned)(set >> 32),
+                                         __builtin_amdgcn_mbcnt_lo((unsigned)set, 0)) << bit;
+        total += __builtin_popcountll(set) << bit;
+      }
+      const unsigned long long hit = __builtin_amdgcn_ballot_w64(pre <= idx && idx < pre + n);
+      if (hit) {  // uniform
+        const int at = __builtin_ffsll((long long)hit) - 1;
+        const int first = __builtin_amdgcn_readlane(pre, at);
+        const int all_steps = __builtin_amdgcn_readlane(steps[w], at);
+        p.b = 64 * w + at;
+        p.len = __builtin_amdgcn_readlane(len[w], at);
+        p.parts = __builtin_amdgcn_readlane(n, at);
+        p.t0 = (idx - first) * all_steps / p.parts;
+        p.tend = (idx - first + 1) * all_steps / p.parts;
+        if (idx == first && p.z == 0 && threadIdx.x == 0)
+          wide_records<RT>(P)[p.b] = make_int2(first, p.parts);
+      }
+      before += total;
+    }
+  return p;
+}
+
 // Wide trees: a workgroup takes RT row tiles of one (request, KV head) and
-// part `part` of its steps (two 32-token tiles each: draft tiles first, then
-// prefix tiles), which its four waves share through LDS, 4 / RT waves on each
-// row tile: with RT = 4 a wave takes both tiles of a step, with RT = 2 one.
-// Each step's K and V go straight into the other of two LDS buffers while
-// the current one is computed, one barrier per step, and hold no registers,
-// so the reads of a whole step's K can be in flight at once.  With one part
-// the rows go to the output, else each part leaves an FP32 partial in slot
-// (row, part) for merge_split_kernel.
+// all of its steps, or with SPLIT the share that wide_part gives it (a step
+// is two 32-token tiles: draft tiles first, then prefix tiles).  Its four
+// waves share the steps through LDS, 4 / RT waves on each row tile: with RT =
+// 4 a wave takes both tiles of a step, with RT = 2 one.  Each step's K and V
+// go straight into the other of two LDS buffers while the current one is
+// computed, one barrier per step, and hold no registers, so the reads of a
+// whole step's K can be in flight at once.  A whole unit's rows go to the
+// output, a share leaves an FP32 partial of each row, in the workgroup's own
+// slots, for merge_wide_kernel.
 // Bound by the matrix units and their clock: 8 requests x 2048 tokens x 256
 // nodes (32/8 heads, D = 128) take 116 us, 594 TFLOP/s (891 with the second
 // MFMA that P's low part takes); the MFMAs alone fill half the cycles, and
 // the clock falls from 2.4 to 1.8 GHz under them.  One 32-token tile per
 // barrier, staged through registers, took 143 us.
-template <int D, int RT>
+template <int D, int RT, bool SPLIT>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreeParams P) {
   constexpr int KS = D / 16;      // MFMA k-steps over the head dimension
   constexpr int DT = D / 32;      // 32-row output tiles over the head dimension
@@ -1312,14 +1429,20 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
   __shared__ uint4 s_anc[BC_MAX_TREE_NODES][2];  // ancestor-or-self set per node, 256 bits
   __shared__ int s_ptr[BC_MAX_TREE_NODES];
 
-  // Workgroup ids put (KV head, row group) in the low bits, then the request,
-  // then the part.
+  // Workgroup ids put (KV head, row group) in the low bits, then the share,
+  // then the request.
   const int rgroups = (P.row_tiles + RT - 1) / RT;
   const int zdim = P.hkv * rgroups;
-  const int unit = blockIdx.x % (zdim * P.batch), part = blockIdx.x / (zdim * P.batch);
-  const int z = unit % zdim, b = unit / zdim;
+  WidePart w{0, 0, 0, 0, 0, 1};
+  if constexpr (SPLIT) {
+    w = wide_part<RT>(P, lane, zdim);
+    if (w.parts == 0) return;  // uniform
+  } else {
+    w.b = blockIdx.x / zdim;
+    w.z = blockIdx.x - w.b * zdim;
+  }
+  const int z = w.z, b = w.b, t0 = w.t0;
   const int kvh = z / rgroups;
-  const int t0 = part * (P.tiles_per_part / TPS);
 
   // First round of loads: the page ids (lane i of a register: entry i of the
   // 64 table entries from step t on, from inside the request's table row),
@@ -1343,10 +1466,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
   }
   const int me = min(tid, P.nodes - 1);
   int up = P.parent[(size_t)b * P.nodes + me];
-  const int len = max(0, min(P.lengths[b], P.max_pages * BC_PAGE_SIZE));
-  const int ntile = ntd + (len + kTile - 1) / kTile;
-  const int tend = min((ntile + TPS - 1) / TPS, t0 + P.tiles_per_part / TPS);
-  if (t0 >= tend) return;  // uniform: the request ends before this part
+  const int len = SPLIT ? w.len : flat_len(P, b);
+  const int tend = SPLIT ? w.tend : (flat_tiles(P, len) + TPS - 1) / TPS;
 
   // Loads: chunk c of a tile is token row (tid + 256c) / CPR, 16 bytes at
   // 8 * (tid % CPR); a wave's chunk lies in one page.
@@ -1435,7 +1556,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
   // steps up, so a chain of any depth (or a cycle) takes at most eight
   // rounds; a serial walk pays one LDS round trip per step of the chain, in
   // every draft tile (2 requests x 333 tokens x a 256-node chain: 88.6 us).
-  if (t0 * TPS < ntd) {  // uniform: the part holds draft tiles
+  if (t0 * TPS < ntd) {  // uniform: the share holds draft tiles
     uint32_t set[8];
 #pragma unroll
     for (int w = 0; w < 8; ++w) set[w] = (me >> 5) == w ? 1u << (me & 31) : 0u;
@@ -1629,10 +1750,10 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
   const size_t orow = ((size_t)b * P.nodes + node) * P.hq + h;
   float* dst = P.out + orow * D;
   float inv = 1.f;
-  if (P.parts == 1) {
+  if (w.parts == 1) {
     inv = 1.f / l;  // every row sees its own node: l > 0
   } else {
-    const size_t slot = orow * P.parts + part;
+    const size_t slot = (size_t)blockIdx.x * (RT * 32) + wrt * 32 + lr;
     dst = P.part_acc + slot * D;
     if (g == 0) *reinterpret_cast<float2*>(P.part_ml + 2 * slot) = make_float2(m, l);
   }
@@ -1645,17 +1766,66 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
                       acc[dt][4 * jq + 2] * inv, acc[dt][4 * jq + 3] * inv);
 }
 
+// Combines the partials of the units that a split launch of tree_wide_kernel
+// cut: one wave per output row (b, node, h).  Lane p holds share p's (max,
+// sum); the weights are formed once and every lane accumulates its dims from
+// the shares, eight at a time.
+template <int D, int RT>
+__global__ __launch_bounds__(256) void merge_wide_kernel(TreeParams P) {
+  pin_params(P);
+  constexpr int PER = D / 64;
+  const int lane = threadIdx.x & 63;
+  const unsigned row =
+      __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));  // (b*N+node)*Hq+h
+  if (row >= (unsigned)P.batch * P.nodes * P.hq) return;
+  const unsigned bn = row / P.hq, h = row - bn * P.hq;
+  const unsigned b = bn / P.nodes, node = bn - b * P.nodes;
+  const int2 rec = wide_records<RT>(P)[b];
+  const int parts = __builtin_amdgcn_readfirstlane(rec.y);
+  if (parts < 2) return;  // written by its only share
+  const int kvh = h / P.group, r = node * P.group + (h - kvh * P.group);
+  const int rgroups = (P.row_tiles + RT - 1) / RT, zdim = P.hkv * rgroups;
+  const int rg = r / (RT * 32);
+  const size_t slot0 =
+      ((size_t)__builtin_amdgcn_readfirstlane(rec.x) * zdim + kvh * rgroups + rg) * (RT * 32) +
+      (r - rg * (RT * 32));
+  const size_t next = (size_t)zdim * (RT * 32);  // from a share's slot to the next one's
+  const float2 ml =
+      *reinterpret_cast<const float2*>(P.part_ml + 2 * (slot0 + min(lane, parts - 1) * next));
+  float x[8][PER], a[PER];
+  auto load = [&](int p0) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const float* src = P.part_acc + (slot0 + min(p0 + u, parts - 1) * next) * D + lane;
+#pragma unroll
+      for (int j = 0; j < PER; ++j) x[u][j] = src[64 * j];
+    }
+  };
+  load(0);
+  const float mp = lane < parts ? ml.x : kNegInf;
+  // Every share holds the row's partial; one of them has its own node, so
+  // the max is finite.
+  const float w = fast_exp2(mp - wave_max(mp));
+  const float lsum = wave_sum(lane < parts ? w * ml.y : 0.f);
+#pragma unroll
+  for (int j = 0; j < PER; ++j) a[j] = 0.f;
+  for (int p0 = 0; p0 < parts; p0 += 8) {
+    if (p0 > 0) load(p0);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (p0 + u < parts) {  // uniform
+        const float wi = __builtin_bit_cast(
+            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), p0 + u));
+#pragma unroll
+        for (int j = 0; j < PER; ++j) a[j] += wi * x[u][j];
+      }
+  }
+  const float inv = 1.f / lsum;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) P.out[(size_t)row * D + lane + 64 * j] = a[j] * inv;
+}
+
 // ---- flat ranges: equal shares of a ragged batch's tiles ----
-
-// Tiles of one (KV head, row tile) of a request of length len: its draft
-// tiles, then its prefix tiles.
-__device__ __forceinline__ int flat_tiles(const TreeParams& P, int len) {
-  return (P.nodes + kTile - 1) / kTile + (len + kTile - 1) / kTile;
-}
-
-__device__ __forceinline__ int flat_len(const TreeParams& P, int b) {
-  return max(0, min(P.lengths[b], P.max_pages * BC_PAGE_SIZE));
-}
 
 __device__ __forceinline__ int wave_incl_scan_i(int x, int lane) {
 #pragma unroll
@@ -2549,39 +2719,42 @@ long long row_groups(const bc_shape& s, int row_tiles, int rt) {
 // tree_split_kernel reads it per row tile, so it takes the trees of several
 // row tiles whose groups fill the CUs (same box, 32/8 heads and D = 128 unless
 // noted, tree_split_kernel or the kernel it replaced first):
-//  - four row tiles a workgroup from 7/8 CUs of groups on: 8 requests x 2048
-//    tokens x 256 nodes 143 against 116 us, 16 x 1000 x 64 nodes 57 against
-//    40, 64 x 30-500 x 64 nodes 73 against 64, 28/4 heads and D = 64: 64 x
-//    1024 x 128 nodes 137 against 118;
+//  - long prefixes (60 tiles), at most one group per CU, and at least 17 steps
+//    per CU in all (D = 64, whose steps are half as long: 24): two workgroups
+//    per CU split the groups by the batch's lengths, four row tiles each (two,
+//    if there are no more).  Against equal parts of the table's capacity: 8 x
+//    128-4096 tokens x 128 nodes 110 -> 67 us, 4 x 500-8000 x 128 88 -> 55, 32
+//    x 256-2048 x 16 48 -> 43, 28/4 heads, D = 64: 16 x 300-3000 x 33 35 ->
+//    31; equal lengths pay 2 to 4 us for finding the share and for the merge
+//    launch: 8 x 2048 x 128 65 -> 69 (103 by tree_split_kernel).  Less work leaves each share too few steps to pay
+//    for its partial rows (16/2 heads: 4 x 4000 x 128 nodes 42 against 46 us,
+//    8 x 2048 x 64 25 against 35; 28/4 heads, D = 64: 28 against 34);
+//  - else four row tiles a workgroup from 7/8 CUs of groups on: 8 requests x
+//    2048 tokens x 256 nodes 143 against 116 us, 16 x 1000 x 64 nodes 57
+//    against 40, 64 x 30-500 x 64 nodes 73 against 64;
 //  - else two a workgroup from two groups per CU on: 64 x 1024 x 9 nodes 50
 //    against 35 us; and from one group per CU on where the prefixes are not
 //    short (30 tiles): 16/16 heads, D = 64: 16 x 1000 x 33 nodes 25 against
 //    20 us, while 28/4 heads, D = 64, 64 x 30-500 x 9 nodes would take 13.2
-//    against 11.2;
-//  - long prefixes (60 tiles) split into parts, two workgroups per CU, from
-//    5/8 CUs of groups on (D = 64, whose tiles are half as long: one): 8 x
-//    128-4096 x 64 nodes 102 against 63 us, 32 x 256-2048 x 16 nodes 59
-//    against 50.  Fewer groups leave each part too few steps to pay for its
-//    partial rows (8 x 2048 x 64 nodes, 16/2 heads: 26 against 31 us).
+//    against 11.2.
 SplitPlan wide_plan(const bc_shape& s, int row_tiles, int max_tiles, int cus) {
   SplitPlan p{0, 0, 4};
   if (row_tiles < 2) return p;
-  const int steps = (max_tiles + 1) / 2;
-  p.parts = 1;
-  p.tiles = 2 * steps;
-  p.wide = 4;
-  if (row_tiles > 2 && 8 * row_groups(s, row_tiles, 4) >= 7LL * cus) return p;
-  const long long u = row_groups(s, row_tiles, 2);
-  p.wide = 2;
-  if (u >= 2LL * cus) return p;
-  if (max_tiles >= 60 && 8 * u >= (s.dim == 64 ? 8LL : 5LL) * cus) {
-    const int parts = (int)(2LL * cus / u);  // 1 to 3
-    const int per = (steps + parts - 1) / parts;
-    p.parts = (steps + per - 1) / per;
-    p.tiles = 2 * per;
+  const int rt = row_tiles > 2 ? 4 : 2;
+  const long long g = row_groups(s, row_tiles, rt);
+  if (max_tiles >= 60 && s.batch <= kWideRequests && g <= cus &&
+      g * max_tiles >= (s.dim == 64 ? 48LL : 34LL) * cus) {
+    p.parts = 2 * cus;
+    p.tiles = cus;
+    p.wide = rt;
     return p;
   }
-  if (max_tiles >= 30 && u >= cus) return p;
+  p.parts = 1;
+  p.wide = 4;
+  if (rt == 4 && 8 * g >= 7LL * cus) return p;
+  const long long u = row_groups(s, row_tiles, 2);
+  p.wide = 2;
+  if (u >= 2LL * cus || (max_tiles >= 30 && u >= cus)) return p;
   p.wide = 0;
   return p;
 }
@@ -2663,9 +2836,10 @@ SplitPlan split_plan(const bc_shape& s, int nodes, int cus) {
 // Workspace of a split plan: P.parts (acc; max, sum) slots per output row.
 size_t split_workspace(const bc_shape& s, int nodes, const SplitPlan& plan, size_t* acc_bytes) {
   if (plan.parts < 2) return 0;
-  const size_t slots = (size_t)s.batch * nodes * s.query_heads * plan.parts;
+  const size_t slots = plan.wide ? (size_t)plan.parts * plan.wide * 32
+                                 : (size_t)s.batch * nodes * s.query_heads * plan.parts;
   *acc_bytes = (slots * s.dim * sizeof(float) + 255) & ~(size_t)255;
-  return *acc_bytes + slots * 2 * sizeof(float);
+  return *acc_bytes + slots * 2 * sizeof(float) + (plan.wide ? s.batch * sizeof(int2) : 0);
 }
 
 template <int D>
@@ -2679,10 +2853,23 @@ void launch_split_kernel(const TreeParams& P, const SplitPlan& plan, dim3 grid,
     tree_split_kernel<D, 8, 1><<<grid, 512, 0, st>>>(P);
 }
 
+template <int D, int RT>
+void launch_wide_kernel(const TreeParams& P, hipStream_t st) {
+  const size_t groups = (size_t)P.batch * P.hkv * ((P.row_tiles + RT - 1) / RT);
+  if (P.parts == 1) {
+    tree_wide_kernel<D, RT, false><<<dim3((unsigned)groups), 256, 0, st>>>(P);
+    return;
+  }
+  tree_wide_kernel<D, RT, true><<<dim3((unsigned)P.parts), 256, 0, st>>>(P);
+  const size_t rows = (size_t)P.batch * P.nodes * P.hq;
+  merge_wide_kernel<D, RT><<<dim3((unsigned)((rows + 3) / 4)), 256, 0, st>>>(P);
+}
+
 template <int D>
-void launch_wide_kernel(const TreeParams& P, const SplitPlan& plan, dim3 grid, hipStream_t st) {
-  if (plan.wide == 2) tree_wide_kernel<D, 2><<<grid, 256, 0, st>>>(P);
-  else tree_wide_kernel<D, 4><<<grid, 256, 0, st>>>(P);
+hipError_t launch_wide(const TreeParams& P, int row_tiles, hipStream_t st) {
+  if (row_tiles == 2) launch_wide_kernel<D, 2>(P, st);
+  else launch_wide_kernel<D, 4>(P, st);
+  return hipGetLastError();
 }
 
 hipError_t launch_split(TreeParams& P, int dim, const SplitPlan& plan, void* workspace,
@@ -2693,21 +2880,15 @@ hipError_t launch_split(TreeParams& P, int dim, const SplitPlan& plan, void* wor
     P.part_acc = static_cast<float*>(workspace);
     P.part_ml = reinterpret_cast<float*>(static_cast<char*>(workspace) + acc_bytes);
   }
-  if (plan.wide) {
-    const size_t groups =
-        (size_t)P.batch * P.hkv * ((P.row_tiles + plan.wide - 1) / plan.wide);
-    const dim3 grid((unsigned)(groups * plan.parts));
-    if (dim == 64) launch_wide_kernel<64>(P, plan, grid, st);
-    else launch_wide_kernel<128>(P, plan, grid, st);
-  } else {
-    const size_t groups = ((size_t)P.batch + plan.rq - 1) / plan.rq;
-    P.grid3d = groups <= 65535;
-    const dim3 grid = P.grid3d
-        ? dim3((unsigned)(P.hkv * P.row_tiles), (unsigned)groups, (unsigned)plan.parts)
-        : dim3((unsigned)((size_t)plan.parts * groups * P.hkv * P.row_tiles));
-    if (dim == 64) launch_split_kernel<64>(P, plan, grid, st);
-    else launch_split_kernel<128>(P, plan, grid, st);
-  }
+  if (plan.wide)
+    return dim == 64 ? launch_wide<64>(P, plan.wide, st) : launch_wide<128>(P, plan.wide, st);
+  const size_t groups = ((size_t)P.batch + plan.rq - 1) / plan.rq;
+  P.grid3d = groups <= 65535;
+  const dim3 grid = P.grid3d
+      ? dim3((unsigned)(P.hkv * P.row_tiles), (unsigned)groups, (unsigned)plan.parts)
+      : dim3((unsigned)((size_t)plan.parts * groups * P.hkv * P.row_tiles));
+  if (dim == 64) launch_split_kernel<64>(P, plan, grid, st);
+  else launch_split_kernel<128>(P, plan, grid, st);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess || plan.parts < 2) return err;
   const size_t rows = (size_t)P.batch * P.nodes * P.hq;
@@ -2782,10 +2963,16 @@ int tree_call(bc_shape s, bc_tree_inputs in, int nodes, void* workspace, size_t 
     const bch::ScratchLease lease(st, need);
     if (lease.get()) return launch_flat(P, s.dim, flat, lease.get(), acc, st);
   }
-  const SplitPlan plan = split_plan(s, nodes, cus);
-  const size_t need = split_workspace(s, nodes, plan, &acc);
+  SplitPlan plan = split_plan(s, nodes, cus);
+  size_t need = split_workspace(s, nodes, plan, &acc);
   if (need == 0) return launch_split(P, s.dim, plan, nullptr, 0, st);
   if (ws_ok && workspace_bytes >= need) return launch_split(P, s.dim, plan, workspace, acc, st);
+  // Four row tiles a workgroup at D = 128 with two workgroups per CU need more
+  // than a slot holds; with one per CU they fit.
+  if (plan.wide == 4 && need > bch::kSlotBytes) {
+    plan.parts = cus;
+    need = split_workspace(s, nodes, plan, &acc);
+  }
   const bch::ScratchLease lease(st, need);
   if (lease.get()) return launch_split(P, s.dim, plan, lease.get(), acc, st);
   // One part per unit.

@@ -2,10 +2,10 @@
 tiles, steps, parts and ranges, against the CPU oracle.
 
 tree_wide_kernel shares K/V tiles between row tiles: two or four a workgroup,
-whole or in parts.  tree_flat_kernel walks equal ranges of a ragged batch's
+whole or split by the batch's lengths.  tree_flat_kernel walks equal ranges of a ragged batch's
 tiles.  Which one a call takes follows from its shape, so each case's shape
 puts it on one of them; short lengths under large page tables keep the oracle
-cheap and leave parts and ranges empty.  The gate is the reference driver's
+cheap and leave shares and ranges uneven or empty.  The gate is the reference driver's
 3e-4 (src/main.cu:505-509).
 """
 
@@ -107,10 +107,16 @@ def _check(fix, oracle, splits):
     (2, 256, 64, 8, 64, 14, False, "malformed"),
     (64, 9, 32, 8, 64, 14, False, "random"),      # two row tiles, two workgroups per CU
     (32, 16, 32, 8, 128, 60, False, "malformed"),  # two, one workgroup per CU
-    (20, 16, 32, 8, 128, 130, True, "random"),    # three parts
-    (32, 16, 32, 8, 128, 130, True, "chain"),     # two parts
+    # Split by the lengths: one long request in many shares, most in one.
+    (20, 16, 32, 8, 128, 130, True, "random"),
+    (32, 16, 32, 8, 128, 130, True, "chain"),
+    (140, 9, 8, 1, 128, 130, True, "malformed"),  # requests in three windows of 64
+    (250, 16, 4, 1, 128, 130, True, "random"),    # in four; more requests than shares to spare
+    (12, 128, 16, 4, 64, 130, True, "chain"),     # shares that begin between draft tiles
     (32, 64, 16, 16, 64, 130, False, "random"),   # D = 64: 512 groups, whole
-    (16, 64, 16, 16, 64, 130, True, "random"),    # D = 64: two parts
+    (16, 64, 16, 16, 64, 130, True, "random"),
+    (16, 33, 28, 4, 64, 190, True, "random"),     # four row tiles a workgroup
+    (8, 64, 32, 8, 128, 190, True, "chain"),      # more than a scratch slot holds
 ])
 def test_wide_trees(batch, nodes, hq, hkv, d, max_pages, splits, parents, oracle):
     fix = _case(batch + nodes, batch, nodes, hq, hkv, d, max_pages, parents=parents,
