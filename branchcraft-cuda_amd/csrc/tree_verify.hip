@@ -1441,20 +1441,25 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
     w.b = blockIdx.x / zdim;
     w.z = blockIdx.x - w.b * zdim;
   }
-  const int z = w.z, b = w.b, t0 = w.t0;
-  const int kvh = z / rgroups;
+  const int b = w.b, t0 = w.t0;
+  const int kvh = w.z / rgroups;
+  int rg = w.z - kvh * rgroups;
+  // Whole units: the later row groups of a tree see more of its draft tiles
+  // (below), so every other round of workgroups over the CUs takes them in the
+  // opposite order.
+  if (!SPLIT && ((b * P.hkv + kvh) * rgroups / P.tiles_per_part) & 1) rg = rgroups - 1 - rg;
 
   // First round of loads: the page ids (lane i of a register: entry i of the
   // 64 table entries from step t on, from inside the request's table row),
   // the row's Q^T fragments (rows past the tree read row (node 0, head 0),
   // whose columns are never written out), the parents and the length.
-  const int ntd = (P.nodes + kTile - 1) / kTile;
+  int ntd = (P.nodes + kTile - 1) / kTile;
   auto load_ids = [&](int t) {
     const int pg = t * PPS - ntd * (kTile / BC_PAGE_SIZE) + lane;
     return P.pages[(size_t)b * P.max_pages + min(max(pg, 0), P.max_pages - 1)];
   };
   int ids = load_ids(t0), ids_next = load_ids(t0 + SPC);
-  const int r = ((z - kvh * rgroups) * RT + wrt) * 32 + lr;
+  const int r = (rg * RT + wrt) * 32 + lr;
   const int rnode = div_by(r, P.group, P.group_mul);
   const int node = r < P.rows ? rnode : 0;
   const int h = kvh * P.group + (r < P.rows ? r - rnode * P.group : 0);
@@ -1467,7 +1472,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
   const int me = min(tid, P.nodes - 1);
   int up = P.parent[(size_t)b * P.nodes + me];
   const int len = SPLIT ? w.len : flat_len(P, b);
-  const int tend = SPLIT ? w.tend : (flat_tiles(P, len) + TPS - 1) / TPS;
+  int tend = SPLIT ? w.tend : (flat_tiles(P, len) + TPS - 1) / TPS;
 
   // Loads: chunk c of a tile is token row (tid + 256c) / CPR, 16 bytes at
   // 8 * (tid % CPR); a wave's chunk lies in one page.
@@ -1579,6 +1584,33 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
         up = s_ptr[up];
       }
       __syncthreads();
+    }
+    // A whole unit ends its draft tiles with the last one that holds an
+    // ancestor of its rows (parents stand before their children, so that is
+    // half of them on average); the two that the first step has loaded stay.
+    // The prefix tiles move up, and their page ids with them.  28 requests x
+    // 14-113 tokens x 221 nodes (32/8 heads, D = 128) 88 -> 71 us, 8 x 2048 x
+    // 256 nodes 120 -> 116.
+    if (!SPLIT && ntd > TPS) {
+      const int r0 = rg * RT * 32, r1 = min(r0 + RT * 32, P.rows) - 1;
+      const int n1 = div_by(r1, P.group, P.group_mul);
+      int last = 0;
+      for (int n0 = div_by(r0, P.group, P.group_mul); n0 <= n1; n0 += 64) {
+        const int n = min(n0 + lane, n1);
+        const uint4 s0 = s_anc[n][0], s1 = s_anc[n][1];
+        const int mine = s1.w ? 7 : s1.z ? 6 : s1.y ? 5 : s1.x ? 4 : s0.w ? 3 : s0.z ? 2 : 0;
+        last = max(last, mine);
+      }
+      int used = TPS;
+#pragma unroll
+      for (int i = TPS; i < 8; ++i) used = __builtin_amdgcn_ballot_w64(last >= i) ? i + 1 : used;
+      const int off = ntd - used;
+      ntd = used;
+      tend = (flat_tiles(P, len) - off + TPS - 1) / TPS;
+      const int from = lane + off * (kTile / BC_PAGE_SIZE);
+      const int lo = __shfl(ids, from & 63, 64), hi = __shfl(ids_next, from & 63, 64);
+      ids = from < 64 ? lo : hi;
+      ids_next = load_ids(SPC);
     }
   }
 
@@ -2341,13 +2373,6 @@ __global__ __launch_bounds__(256) void merge_flat_kernel(TreeParams P) {
         make_float4(a[j].x * inv, a[j].y * inv, a[j].z * inv, a[j].w * inv);
 }
 
-// Wide trees: RT row tiles of a (request, KV head) per workgroup (four
-// waves, 4 / RT of them on each row tile), which share every K/V tile
-// through LDS.  A step is two 32-token tiles; with RT = 4 each wave takes
-// both, with RT = 2 one of them.  Steps form flat ranges as in
-// tree_flat_kernel.  Each step's loads are issued a step ahead into
-// registers and staged into the other LDS buffer after the step's math, one
-// barrier per step.
 // Row-sharing variant, for tensors that are not 16-byte aligned, of trees of
 // four or more row tiles per (request, KV head), where tree_kernel would read
 // the prefix once per row tile: the four
@@ -2704,7 +2729,7 @@ bool tree_ptrs_aligned(const bc_tree_inputs& in) {
 
 struct SplitPlan {
   int parts;  // workgroups per (request group, KV head, row tile), <= 64
-  int tiles;  // 32-token tiles per workgroup and request (draft then prefix tiles)
+  int tiles;  // 32-token tiles per workgroup and request (draft then prefix tiles); wide: CUs
   int waves;  // waves per workgroup: 4 or 8
   int rq = 1;  // requests per workgroup (waves / rq per request)
   int wide = 0;  // row tiles per workgroup of tree_wide_kernel (0: tree_split_kernel)
@@ -2750,6 +2775,7 @@ SplitPlan wide_plan(const bc_shape& s, int row_tiles, int max_tiles, int cus) {
     return p;
   }
   p.parts = 1;
+  p.tiles = cus;
   p.wide = 4;
   if (rt == 4 && 8 * g >= 7LL * cus) return p;
   const long long u = row_groups(s, row_tiles, 2);
@@ -2980,7 +3006,8 @@ int tree_call(bc_shape s, bc_tree_inputs in, int nodes, void* workspace, size_t 
       (s.max_pages * BC_PAGE_SIZE + kTile - 1) / kTile + (nodes + kTile - 1) / kTile;
   SplitPlan one{1, (max_tiles + 1) / 2 * 2, 8};
   one.wide = plan.wide;
-  if (!one.wide)
+  if (one.wide) one.tiles = cus;
+  else
     one = pair_requests(P.batch, (long long)P.batch * P.hkv * P.row_tiles, one, cus);
   return launch_split(P, s.dim, one, nullptr, 0, st);
 }

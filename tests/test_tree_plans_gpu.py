@@ -105,6 +105,12 @@ def _check(fix, oracle, splits):
     (32, 100, 28, 4, 64, 14, False, "random"),    # group 7: 22 row tiles, partly filled rows
     (7, 256, 32, 8, 128, 14, False, "chain"),     # the widest tree: eight draft tiles
     (2, 256, 64, 8, 64, 14, False, "malformed"),
+    # Draft tiles that no row of a row group sees: a group of 128 nodes, one
+    # with its last ancestors in the first tile of a window, and odd counts.
+    (40, 256, 8, 8, 64, 14, False, "random"),
+    (40, 129, 8, 8, 128, 14, False, "malformed"),
+    (28, 97, 28, 4, 128, 60, False, "chain"),
+    (28, 65, 32, 8, 128, 58, False, "random"),
     (64, 9, 32, 8, 64, 14, False, "random"),      # two row tiles, two workgroups per CU
     (32, 16, 32, 8, 128, 60, False, "malformed"),  # two, one workgroup per CU
     # Split by the lengths: one long request in many shares, most in one.
