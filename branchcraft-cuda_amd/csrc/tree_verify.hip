@@ -1778,24 +1778,55 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
         acc[dt][4 * jq + 3] = acc[dt][4 * jq + 3] * a1 + v4.w * a2;
       }
   }
-  if (r >= P.rows) return;
-  const size_t orow = ((size_t)b * P.nodes + node) * P.hq + h;
-  float* dst = P.out + orow * D;
   float inv = 1.f;
+  float* to = P.out;
+  size_t idx = ((size_t)b * P.nodes + node) * P.hq + h;  // this lane's row of `to`
   if (w.parts == 1) {
     inv = 1.f / l;  // every row sees its own node: l > 0
   } else {
-    const size_t slot = (size_t)blockIdx.x * (RT * 32) + wrt * 32 + lr;
-    dst = P.part_acc + slot * D;
-    if (g == 0) *reinterpret_cast<float2*>(P.part_ml + 2 * slot) = make_float2(m, l);
+    to = P.part_acc;
+    idx = (size_t)blockIdx.x * (RT * 32) + wrt * 32 + lr;
+    if (g == 0 && r < P.rows) *reinterpret_cast<float2*>(P.part_ml + 2 * idx) = make_float2(m, l);
   }
+  if constexpr (TS > 1) {
+    if (r >= P.rows) return;
+    float* dst = to + idx * D;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq)
+        *reinterpret_cast<float4*>(dst + 32 * dt + 8 * jq + 4 * g) =
+            make_float4(acc[dt][4 * jq] * inv, acc[dt][4 * jq + 1] * inv,
+                        acc[dt][4 * jq + 2] * inv, acc[dt][4 * jq + 3] * inv);
+    return;
+  }
+  // Rows leave through LDS, each wave's in its own part of the staged tiles
+  // (all read by now), so that a store covers whole rows; stored from the
+  // accumulators, as where only half of the waves have rows to write (64 x
+  // 1024 tokens x 9 nodes: 48.8 us, 49.2 through LDS), it writes 32 bytes of
+  // each of 32 rows.  41 x 48-97 tokens x 137 nodes (28/4 heads, D = 128) 60.9
+  // -> 57.3 us, 31 x 30-61 x 100 (32/8, D = 64) 25.0 -> 23.8, partials of 8 x
+  // 4096 x 64 (32/8, D = 128) 70.3 -> 67.0.
+  static_assert(RT * 32 * D * 4 <= sizeof(s_kv), "the rows fit the staged tiles");
+  float* const mine = reinterpret_cast<float*>(s_kv[0]) + wrt * 32 * D;
+  constexpr int C4 = D / 4;  // four-float chunks per row, chunk c of row i at c ^ (i % C4)
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int jq = 0; jq < 4; ++jq)
-      *reinterpret_cast<float4*>(dst + 32 * dt + 8 * jq + 4 * g) =
+      *reinterpret_cast<float4*>(mine + lr * D + (((8 * dt + 2 * jq + g) ^ (lr % C4)) << 2)) =
           make_float4(acc[dt][4 * jq] * inv, acc[dt][4 * jq + 1] * inv,
                       acc[dt][4 * jq + 2] * inv, acc[dt][4 * jq + 3] * inv);
+  wave_lds_sync();
+  const int nrow = P.rows - (rg * RT + wrt) * 32;  // valid rows, from the first one on
+  constexpr int RPS = 64 / C4;                     // rows per store
+#pragma unroll
+  for (int i = 0; i < 32; i += RPS) {
+    const int row = i + lane / C4, c = lane % C4;
+    const float4 v = *reinterpret_cast<const float4*>(mine + row * D + ((c ^ (row % C4)) << 2));
+    const size_t at = __shfl((unsigned long long)idx, row, 64);
+    if (row < nrow) *reinterpret_cast<float4*>(to + at * D + 4 * c) = v;
+  }
 }
 
 // Combines the partials of the units that a split launch of tree_wide_kernel
