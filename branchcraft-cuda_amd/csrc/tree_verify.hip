@@ -1561,7 +1561,26 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
   // steps up, so a chain of any depth (or a cycle) takes at most eight
   // rounds; a serial walk pays one LDS round trip per step of the chain, in
   // every draft tile (2 requests x 333 tokens x a 256-node chain: 88.6 us).
-  if (t0 * TPS < ntd) {  // uniform: the share holds draft tiles
+  if (t0 * TPS < ntd && P.nodes <= 64) {
+    // One node per lane of the first wave: no LDS and no barrier a round (64 x
+    // 8-64 tokens x 33 nodes, 32/8 heads, D = 128: 29.0 -> 26.1 us; 64 x 16-128
+    // x 64, D = 64: 24.8 -> 21.8).  The barrier below publishes the sets.
+    if (wave == 0) {
+      uint32_t set0 = lane < 32 ? 1u << lane : 0u, set1 = lane < 32 ? 0u : 1u << (lane - 32);
+      if (lane >= P.nodes || up < 0 || up >= P.nodes) up = -1;
+      for (int round = 0; round < 6 && __builtin_amdgcn_ballot_w64(up >= 0); ++round) {
+        const int from = max(up, 0);
+        const uint32_t a0 = __shfl(set0, from, 64), a1 = __shfl(set1, from, 64);
+        const int next = __shfl(up, from, 64);
+        if (up >= 0) {
+          set0 |= a0;
+          set1 |= a1;
+          up = next;
+        }
+      }
+      s_anc[lane][0] = make_uint4(set0, set1, 0, 0);
+    }
+  } else if (t0 * TPS < ntd) {  // uniform: the share holds draft tiles
     uint32_t set[8];
 #pragma unroll
     for (int w = 0; w < 8; ++w) set[w] = (me >> 5) == w ? 1u << (me & 31) : 0u;

@@ -113,6 +113,11 @@ def _check(fix, oracle, splits):
     (28, 65, 32, 8, 128, 58, False, "random"),
     (64, 9, 32, 8, 64, 14, False, "random"),      # two row tiles, two workgroups per CU
     (32, 16, 32, 8, 128, 60, False, "malformed"),  # two, one workgroup per CU
+    # The ancestor sets of one wave: 64 nodes, one short of them, chains and
+    # cycles over all of them.
+    (30, 64, 32, 8, 128, 14, False, "chain"),
+    (30, 63, 32, 8, 64, 14, False, "malformed"),
+    (30, 64, 32, 8, 64, 14, False, "malformed"),
     # Split by the lengths: one long request in many shares, most in one.
     (20, 16, 32, 8, 128, 130, True, "random"),
     (32, 16, 32, 8, 128, 130, True, "chain"),
