@@ -1294,7 +1294,7 @@ constexpr int kWideStep = 2 * kTile;     // tokens per step
 constexpr int kWideRequests = 4 * 64;    // requests of a split launch, four per lane
 constexpr int kWideParts = 63;           // most shares of a unit
 constexpr int kWideLeast = 6;            // fewest steps per share of a long unit
-constexpr float kWideSlack = 12.f;       // steps that a batch's partials cost
+constexpr float kWideSlack = 11.f;       // steps that a batch's partials cost
 
 // Per request: the first of its shares in the launch's order, and how many.
 // They stand after the partials' (max, sum) pairs.
@@ -1335,9 +1335,15 @@ __device__ __forceinline__ WidePart wide_part(const TreeParams& P, int lane, int
   };
   int per = max(max((all + cap - 1) / cap, (longest + kWideParts - 1) / kWideParts),
                 kWideLeast);
-  // An even batch (equal lengths, most CUs with a unit) gains nothing that
-  // its partials would not cost: whole units.
-  if ((float)longest <= (float)all * (float)zdim / (float)P.tiles_per_part + kWideSlack)
+  // An even batch (equal lengths, most CUs with a unit) runs whole units, one
+  // per CU, unless they are long: two workgroups per CU hide a fifth of the
+  // steps behind each other, and a batch's partials cost about kWideSlack
+  // steps.  Whole against shares, 32/8 heads and D = 128 unless noted: 8 x 2048
+  // x 128 nodes 69.6 against 71.2 us, 30 x 2048 x 32 72.9 against 76.7; 57 x
+  // 3696 x 11 (28/4 heads) 129 against 114, 8 x 8000 x 128 217 against 206, 28
+  // x 6000 x 48 (16/4, D = 64) 111 against 94, 16 x 4096 x 64 (D = 64) 83
+  // against 79.
+  if (1.2f * (float)longest <= (float)all * (float)zdim / (float)P.tiles_per_part + kWideSlack)
     per = max(per, longest);
   for (int hi = max(per, longest); per < hi;) {
     const int mid = (per + hi) >> 1;

@@ -128,6 +128,7 @@ def _check(fix, oracle, splits):
     (16, 64, 16, 16, 64, 130, True, "random"),
     (16, 33, 28, 4, 64, 190, True, "random"),     # four row tiles a workgroup
     (8, 64, 32, 8, 128, 190, True, "chain"),      # more than a scratch slot holds
+    (28, 40, 16, 4, 64, 190, True, "random"),     # an even batch but for one long request
 ])
 def test_wide_trees(batch, nodes, hq, hkv, d, max_pages, splits, parents, oracle):
     fix = _case(batch + nodes, batch, nodes, hq, hkv, d, max_pages, parents=parents,
