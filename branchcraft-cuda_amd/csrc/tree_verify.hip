@@ -2818,12 +2818,13 @@ long long row_groups(const bc_shape& s, int row_tiles, int rt) {
 //    short (30 tiles): 16/16 heads, D = 64: 16 x 1000 x 33 nodes 25 against
 //    20 us, while 28/4 heads, D = 64, 64 x 30-500 x 9 nodes would take 13.2
 //    against 11.2.
-SplitPlan wide_plan(const bc_shape& s, int row_tiles, int max_tiles, int cus) {
+// Without scratch memory (`scratch` false) there is no split.
+SplitPlan wide_plan(const bc_shape& s, int row_tiles, int max_tiles, int cus, bool scratch) {
   SplitPlan p{0, 0, 4};
   if (row_tiles < 2) return p;
   const int rt = row_tiles > 2 ? 4 : 2;
   const long long g = row_groups(s, row_tiles, rt);
-  if (max_tiles >= 60 && s.batch <= kWideRequests && g <= cus &&
+  if (scratch && max_tiles >= 60 && s.batch <= kWideRequests && g <= cus &&
       g * max_tiles >= (s.dim == 64 ? 48LL : 34LL) * cus) {
     p.parts = 2 * cus;
     p.tiles = cus;
@@ -2888,7 +2889,7 @@ SplitPlan split_plan(const bc_shape& s, int nodes, int cus) {
     return parts < 2 ? p : SplitPlan{parts, tiles, waves};
   };
   const long long u = units > 0 ? units : 1;
-  const SplitPlan wide = wide_plan(s, row_tiles, max_tiles, cus);
+  const SplitPlan wide = wide_plan(s, row_tiles, max_tiles, cus, true);
   if (wide.wide) return wide;
   // A single pass whose eight waves take two tiles or fewer each beats a
   // split, which adds the merge launch (one request over 256 tokens: 8.2
@@ -3057,14 +3058,14 @@ int tree_call(bc_shape s, bc_tree_inputs in, int nodes, void* workspace, size_t 
   }
   const bch::ScratchLease lease(st, need);
   if (lease.get()) return launch_split(P, s.dim, plan, lease.get(), acc, st);
-  // One part per unit.
+  // One part per unit, by the rules for whole units: few wide ones would leave
+  // most CUs idle.
   const int max_tiles =
       (s.max_pages * BC_PAGE_SIZE + kTile - 1) / kTile + (nodes + kTile - 1) / kTile;
-  SplitPlan one{1, (max_tiles + 1) / 2 * 2, 8};
-  one.wide = plan.wide;
-  if (one.wide) one.tiles = cus;
-  else
-    one = pair_requests(P.batch, (long long)P.batch * P.hkv * P.row_tiles, one, cus);
+  SplitPlan one = wide_plan(s, P.row_tiles, max_tiles, cus, false);
+  if (!one.wide)
+    one = pair_requests(P.batch, (long long)P.batch * P.hkv * P.row_tiles,
+                        SplitPlan{1, (max_tiles + 1) / 2 * 2, 8}, cus);
   return launch_split(P, s.dim, one, nullptr, 0, st);
 }
 

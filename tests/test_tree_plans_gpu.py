@@ -62,7 +62,7 @@ def _case(seed, batch, nodes, hq, hkv, d, max_pages, pool=None, longest=0, paren
     return k, v, pages, lengths, dq, dk, dv, par.astype(np.int32)
 
 
-def _run(fix, workspace):
+def _run(fix, workspace, captured=False):
     k, v, pages, lengths, dq, dk, dv, par = fix
     b, n, hq, d = dq.shape
     shape = capi.Shape(b, hq, k.shape[2], d, pages.shape[1], k.shape[0])
@@ -76,6 +76,18 @@ def _run(fix, workspace):
         nbytes = L.bc_tree_verify_workspace_size(shape, n)
         ws = torch.full((max(1, nbytes),), 0xff, device="cuda", dtype=torch.uint8)  # NaN partials
         G.check(L.bc_tree_verify_ws(shape, ins, n, ws.data_ptr(), nbytes, G.stream()), "ws call")
+    elif captured:
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            G.check(L.bc_tree_verify(shape, ins, n, G.stream()), "captured call")
+        replays = []
+        for _ in range(3):
+            out.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            replays.append(out.clone())
+        assert all(torch.equal(x, replays[0]) for x in replays)
     else:
         G.check(L.bc_tree_verify(shape, ins, n, G.stream()), "call")
     torch.cuda.synchronize()
@@ -134,6 +146,19 @@ def test_wide_trees(batch, nodes, hq, hkv, d, max_pages, splits, parents, oracle
     fix = _case(batch + nodes, batch, nodes, hq, hkv, d, max_pages, parents=parents,
                 longest=1500 if max_pages > 100 else 0)
     _check(fix, oracle, splits)
+
+
+@pytest.mark.parametrize("batch,nodes,hq,hkv,d,max_pages", [
+    (12, 128, 16, 4, 64, 130),  # few wide units: a row tile a workgroup
+    (32, 16, 32, 8, 128, 130),  # one per CU: whole wide units
+])
+def test_split_shapes_under_capture(batch, nodes, hq, hkv, d, max_pages, oracle):
+    """A captured call without a workspace has no scratch and runs whole units."""
+    fix = _case(3, batch, nodes, hq, hkv, d, max_pages, longest=1500)
+    k, v, pages, lengths, dq, dk, dv, par = fix
+    expected = oracle.tree(k.cpu().numpy(), v.cpu().numpy(), pages, lengths, dq, dk, dv, par,
+                           threads=16)
+    G.gate(_run(fix, False, captured=True), expected, 3e-4, "captured")
 
 
 @pytest.mark.parametrize("batch,nodes,hq,hkv,d,max_pages,pool,longest,parents", [
