@@ -2810,6 +2810,15 @@ long long row_groups(const bc_shape& s, int row_tiles, int rt) {
 //    launch: 8 x 2048 x 128 65 -> 69 (103 by tree_split_kernel).  Less work leaves each share too few steps to pay
 //    for its partial rows (16/2 heads: 4 x 4000 x 128 nodes 42 against 46 us,
 //    8 x 2048 x 64 25 against 35; 28/4 heads, D = 64: 28 against 34);
+//    but prefixes of more than 32 MB, which the eight L2s do not hold, cost
+//    tree_split_kernel a trip past the L2 per row tile, and from 5 steps per CU
+//    (D = 64: 12) the shares win: 14 x 2319 x 32 nodes 86 against 47 us, 9 x
+//    450-3600 x 32 (32/4) 74 against 38, 6 x 1079-2158 x 12 (24/8) 22.3 against
+//    19.3, 22 x 1934 x 9 (16/2) 28.5 against 27.2, D = 64: 21 x 2333 x 16 (28/4)
+//    36 against 27; fewer steps: 10 x 1041-2082 x 20 (D = 64) 22.0 against 24.3.
+//    On prefixes that do not reach it, shared by the requests or few, the rule
+//    above stays: 16 x 2454 x 16 (24/8, D = 64, one shared prefix) 18 against
+//    23, 5 x 2102 x 33 (32/4, shared) 22 against 32;
 //  - else four row tiles a workgroup from 7/8 CUs of groups on: 8 requests x
 //    2048 tokens x 256 nodes 143 against 116 us, 16 x 1000 x 64 nodes 57
 //    against 40, 64 x 30-500 x 64 nodes 73 against 64;
@@ -2824,8 +2833,13 @@ SplitPlan wide_plan(const bc_shape& s, int row_tiles, int max_tiles, int cus, bo
   if (row_tiles < 2) return p;
   const int rt = row_tiles > 2 ? 4 : 2;
   const long long g = row_groups(s, row_tiles, rt);
+  const long long page = 2LL * BC_PAGE_SIZE * s.kv_heads * s.dim * sizeof(uint16_t);
+  // The prefixes' bytes, as far as the shape tells, against eight L2s of 4 MB.
+  const bool far =
+      std::min((long long)s.batch * s.max_pages, (long long)s.physical_pages) * page > 32000000;
+  const long long least = s.dim == 64 ? (far ? 24LL : 48LL) : (far ? 10LL : 34LL);
   if (scratch && max_tiles >= 60 && s.batch <= kWideRequests && g <= cus &&
-      g * max_tiles >= (s.dim == 64 ? 48LL : 34LL) * cus) {
+      g * max_tiles >= least * cus) {
     p.parts = 2 * cus;
     p.tiles = cus;
     p.wide = rt;

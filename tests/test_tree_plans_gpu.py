@@ -148,6 +148,19 @@ def test_wide_trees(batch, nodes, hq, hkv, d, max_pages, splits, parents, oracle
     _check(fix, oracle, splits)
 
 
+@pytest.mark.parametrize("batch,nodes,hq,hkv,d,max_pages,pool,parents", [
+    (9, 32, 32, 4, 128, 226, 2040, "random"),   # a pool past the L2s
+    (6, 12, 24, 8, 128, 136, 800, "chain"),     # two row tiles
+    (21, 16, 28, 4, 64, 147, 3080, "malformed"),
+    (3, 33, 64, 8, 128, 165, 520, "random"),    # nine row tiles
+    (9, 32, 32, 4, 128, 226, 0, "chain"),       # the same shape, a small pool
+])
+def test_wide_trees_over_large_pools(batch, nodes, hq, hkv, d, max_pages, pool, parents, oracle):
+    fix = _case(batch + nodes, batch, nodes, hq, hkv, d, max_pages, pool=pool, parents=parents,
+                longest=2000)
+    _check(fix, oracle, True)
+
+
 @pytest.mark.parametrize("batch,nodes,hq,hkv,d,max_pages", [
     (12, 128, 16, 4, 64, 130),  # few wide units: a row tile a workgroup
     (32, 16, 32, 8, 128, 130),  # one per CU: whole wide units
