@@ -1404,7 +1404,7 @@ __device__ __forceinline__ WidePart wide_part(const TreeParams& P, int lane, int
 // output, a share leaves an FP32 partial of each row, in the workgroup's own
 // slots, for merge_wide_kernel.
 // Bound by the matrix units and their clock: 8 requests x 2048 tokens x 256
-// nodes (32/8 heads, D = 128) take 116 us, 594 TFLOP/s (891 with the second
+// nodes (32/8 heads, D = 128) take 112 us, 617 TFLOP/s (925 with the second
 // MFMA that P's low part takes); the MFMAs alone fill half the cycles, and
 // the clock falls from 2.4 to 1.8 GHz under them.  One 32-token tile per
 // barrier, staged through registers, took 143 us.
