@@ -70,20 +70,19 @@ class PagedTreeCache:
         kernel arguments.  What the op does not take -- a pool that is not on
         the GPU, rows that autograd tracks, a subclass, or rows that are views
         of the pool itself -- is copied page by page."""
-        store = [x.untyped_storage().data_ptr() for x in (self.k, self.v)]
-        rows = []
-        for x in (prefix_k, prefix_v):
-            if (not self.k.is_cuda or type(x) not in (torch.Tensor, torch.nn.Parameter)
-                    or (x.requires_grad and torch.is_grad_enabled())
-                    or x.untyped_storage().data_ptr() in store):
-                break
-            # V of another type or device is converted as a copy would.
-            x = x.to(self.k.device, torch.float16)
-            rows.append(x if x.stride(-1) == 1 else x.contiguous())
-        else:
-            if pages:
-                write_prefix_(self.k, self.v, *rows, pages)
-            return
+        if self.k.is_cuda and type(self.k) is torch.Tensor and all(
+                type(x) in (torch.Tensor, torch.nn.Parameter)
+                and not (x.requires_grad and torch.is_grad_enabled())
+                for x in (prefix_k, prefix_v)):
+            store = [x.untyped_storage().data_ptr() for x in (self.k, self.v)]
+            rows = [prefix_k, prefix_v]
+            if not any(x.untyped_storage().data_ptr() in store for x in rows):
+                # V of another type or device is converted as a copy would.
+                rows = [x.to(self.k.device, torch.float16) for x in rows]
+                rows = [x if x.stride(-1) == 1 else x.contiguous() for x in rows]
+                if pages:
+                    write_prefix_(self.k, self.v, *rows, pages)
+                return
         for i, page in enumerate(pages):
             n = min(16, prefix_k.shape[0] - 16 * i)
             self.k[page, :n].copy_(prefix_k[16 * i:16 * i + n])
@@ -104,14 +103,15 @@ class PagedTreeCache:
     def _upload(self, *lists) -> tuple[torch.Tensor, ...]:
         """The lists as int32 tensors on the pool's device, all of them parts
         of one.  The values go in kernel arguments; a pool that is not on the
-        GPU, entries that are not plain integers, and a stream under capture,
+        GPU or holds no memory at all (fake tensors, also on a machine without
+        a GPU), entries that are not plain integers, and a stream under capture,
         where the values would be frozen into the graph and a copy raises
         instead, take a copy from host memory.  A step of eight requests of 2053
         tokens (eight verify calls, one commit_many, rollbacks) takes 335 us,
         611 with a copy per list and page-by-page bookkeeping."""
         values = [x for part in lists for x in part]
-        if (self.k.is_cuda and set(map(type, values)) == {int}
-                and not torch.cuda.is_current_stream_capturing()):
+        if (self.k.is_cuda and type(self.k) is torch.Tensor
+                and set(map(type, values)) == {int} and not torch.cuda.is_current_stream_capturing()):
             flat = int_tensor(self.k, values)
         else:
             flat = torch.tensor(values, dtype=torch.int32).to(self.k.device)

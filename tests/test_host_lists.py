@@ -132,3 +132,30 @@ def test_runs_of_pages_stop_where_single_pages_do():
     with pytest.raises(RuntimeError, match="free list holds referenced page 1"):
         owner.new(48)
     assert owner.refcount == [1, 1, 0, 0] and owner.free == [3, 2]
+
+
+@pytest.mark.parametrize("device", ["cuda", "cpu", "meta"])
+def test_transaction_on_fake_tensors(device):
+    """Shapes of a whole transaction without memory, and for device "cuda"
+    without a GPU; no warning about a fake tensor's address."""
+    import warnings
+
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from branchcraft_torch.transaction import PagedTreeCache
+    with FakeTensorMode(), warnings.catch_warnings():
+        warnings.simplefilter("error")
+
+        def half(*shape):
+            return torch.empty(shape, device=device, dtype=torch.float16)
+
+        cache = PagedTreeCache(20, 2, 64, device=device)
+        one = cache.new(half(19, 2, 64), half(19, 2, 64))
+        two = cache.fork(one)
+        dk = half(1, 3, 2, 64)
+        parent = torch.zeros((1, 3), device=device, dtype=torch.int32)
+        out = cache.verify(one, half(1, 3, 4, 64), dk, dk, parent)
+        assert out.shape == (1, 3, 4, 64) and out.dtype == torch.float32
+        assert cache.commit(one, [0, 2], dk, dk).cow == (1, 2)
+        assert cache.commit_many([two, one], [[1], [0]], dk.expand(2, 3, 2, 64),
+                                 dk.expand(2, 3, 2, 64))[0].cow is None
+        assert cache.lengths == {one: 22, two: 20}
