@@ -366,6 +366,21 @@ void write_prefix_hip(at::Tensor& cache_k, at::Tensor& cache_v, const at::Tensor
                "write_prefix_");
 }
 
+// Above the kernel: the pools' version counters move, so that a backward that
+// saved a pool before a prompt entered it raises, as after slice copies.
+void write_prefix_versioned(at::Tensor& cache_k, at::Tensor& cache_v, const at::Tensor& k,
+                            const at::Tensor& v, at::IntArrayRef pages) {
+  static const auto op =
+      c10::Dispatcher::singleton()
+          .findSchemaOrThrow("branchcraft::write_prefix_", "")
+          .typed<void(at::Tensor&, at::Tensor&, const at::Tensor&, const at::Tensor&,
+                      at::IntArrayRef)>();
+  cache_k.unsafeGetTensorImpl()->bump_version();
+  cache_v.unsafeGetTensorImpl()->bump_version();
+  const at::AutoDispatchBelowADInplaceOrView below;
+  op.call(cache_k, cache_v, k, v, pages);
+}
+
 // A host list as an int32 tensor on `like`'s device, written in stream order
 // by kernels that carry the values as arguments.
 at::Tensor int_tensor_hip(const at::Tensor& like, at::IntArrayRef values) {
@@ -408,4 +423,8 @@ TORCH_LIBRARY_IMPL(branchcraft, CUDA, m) {
   m.impl("write_prefix_", write_prefix_hip);
   m.impl("int_tensor", int_tensor_hip);
   m.impl("paged_decode", paged_decode_hip);
+}
+
+TORCH_LIBRARY_IMPL(branchcraft, ADInplaceOrView, m) {
+  m.impl("write_prefix_", write_prefix_versioned);
 }

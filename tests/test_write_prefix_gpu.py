@@ -84,3 +84,36 @@ def test_new_on_a_host_pool_copies_by_page():
     pages = store.pages[store.new(k, v)]
     assert torch.equal(store.k, _by_page(torch.zeros_like(store.k), k, pages))
     assert torch.equal(store.v, _by_page(torch.zeros_like(store.v), v, pages))
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_write_prefix_moves_the_version_counters(grad):
+    """Once per call, on the pools alone; fake tensors, so that it runs
+    without a GPU.  An inference pool is refused outside inference mode, as
+    an in-place copy into it is."""
+    import branchcraft_torch as bt
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode(), torch.set_grad_enabled(grad):
+        pools = [torch.zeros(4, 16, 2, 64, device="cuda", dtype=torch.float16) for _ in range(2)]
+        rows = [torch.zeros(19, 2, 64, device="cuda", dtype=torch.float16) for _ in range(2)]
+        for calls in (1, 2):
+            bt.write_prefix_(*pools, *rows, [2, 0])
+            assert [x._version for x in pools + rows] == [calls, calls, 0, 0]
+        with torch.inference_mode():
+            frozen = [x.clone() for x in pools]
+            bt.write_prefix_(*frozen, *rows, [2, 0])
+        with pytest.raises(RuntimeError, match="inference tensor"):
+            bt.write_prefix_(*frozen, *rows, [2, 0])
+
+
+@pytest.mark.gpu
+def test_backward_sees_a_prompt_enter_the_pool():
+    """A pool saved for backward before ``new`` has other values after it."""
+    from branchcraft_torch.transaction import PagedTreeCache
+    store = PagedTreeCache(4, 2, 64)
+    rows = torch.randn(19, 2, 64, device="cuda", dtype=torch.float16)
+    x = torch.ones((), device="cuda", dtype=torch.float16, requires_grad=True)
+    y = (store.k * x).sum()
+    store.new(rows, rows)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward()
