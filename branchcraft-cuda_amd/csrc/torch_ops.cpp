@@ -355,8 +355,12 @@ void write_prefix_hip(at::Tensor& cache_k, at::Tensor& cache_v, const at::Tensor
   TORCH_CHECK(cache_k.device() == cache_v.device() && cache_k.device() == k.device() &&
                   cache_k.device() == v.device(),
               "all tensors must share a device");
+  TORCH_CHECK(k.size(0) <= INT32_MAX, "write_prefix_: too many tokens");
   const c10::DeviceGuard guard(cache_k.device());
-  c10::SmallVector<int32_t, 512> ids(pages.begin(), pages.end());
+  // Ids past 32 bits are outside every pool, and skipped as such.
+  c10::SmallVector<int32_t, 512> ids(pages.size());
+  for (size_t i = 0; i < pages.size(); ++i)
+    ids[i] = pages[i] >= 0 && pages[i] <= INT32_MAX ? int32_t(pages[i]) : -1;
   bc_shape shape{1, int(cache_k.size(2)), int(cache_k.size(2)), int(cache_k.size(3)), 1,
                  int(cache_k.size(0))};
   if (k.size(0) == 0) return;

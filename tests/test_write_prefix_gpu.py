@@ -117,3 +117,17 @@ def test_backward_sees_a_prompt_enter_the_pool():
     store.new(rows, rows)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         y.backward()
+
+
+@pytest.mark.gpu
+def test_page_ids_past_32_bits_are_skipped():
+    """As other ids outside the pool: none of them names a page by its low
+    bits."""
+    import branchcraft_torch as bt
+    pools = [torch.zeros(8, 16, 2, 64, device="cuda", dtype=torch.float16) for _ in range(2)]
+    rows = torch.randn(16 * 6, 2, 64, device="cuda", dtype=torch.float16)
+    pages = [2**32 + 1, 2, -2**32 + 3, 2**63 - 1, -2**63, 8]
+    want = torch.zeros_like(pools[0])
+    want[2] = rows[16:32]
+    bt.write_prefix_(*pools, rows, rows, pages)
+    assert all(torch.equal(x, want) for x in pools)
