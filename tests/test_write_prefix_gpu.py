@@ -131,3 +131,34 @@ def test_page_ids_past_32_bits_are_skipped():
     want[2] = rows[16:32]
     bt.write_prefix_(*pools, rows, rows, pages)
     assert all(torch.equal(x, want) for x in pools)
+
+
+@pytest.mark.gpu
+def test_new_under_autograd_is_what_slice_copies_are():
+    """A leaf pool is refused, a tracked pool keeps its graph (a row that a
+    later prompt overwrites gets no gradient), and a tangent reaches the pool."""
+    import torch.autograd.forward_ad as fw
+    from branchcraft_torch.transaction import PagedTreeCache
+    k = torch.randn(32, 2, 64, device="cuda", dtype=torch.float16)
+    store = PagedTreeCache(4, 2, 64)
+    store.k.requires_grad_()
+    with pytest.raises(RuntimeError, match="leaf Variable"):
+        store.new(k, k)
+    for tracked in ("k", "v"):
+        store, rows = PagedTreeCache(4, 2, 64), k.clone().requires_grad_()
+        first = store.new(*((rows, k) if tracked == "k" else (k, rows)))
+        for page in reversed(store.pages.pop(first)):
+            store.owner.release(page)
+        store.new(k[:16], k[:16])  # over the first page
+        getattr(store, tracked).sum().backward()
+        assert torch.equal(rows.grad[:16], torch.zeros_like(k[:16]))
+        assert torch.equal(rows.grad[16:], torch.ones_like(k[16:]))
+    for at in range(2):
+        with fw.dual_level():
+            store = PagedTreeCache(4, 2, 64)
+            pair = [k, k]
+            pair[at] = fw.make_dual(k, 2 * k)
+            store.new(*pair)
+            tangents = [fw.unpack_dual(x).tangent for x in (store.k, store.v)]
+            assert tangents[1 - at] is None
+            assert torch.equal(tangents[at][:2].reshape(32, 2, 64), 2 * k)
