@@ -370,10 +370,25 @@ void write_prefix_hip(at::Tensor& cache_k, at::Tensor& cache_v, const at::Tensor
                "write_prefix_");
 }
 
-// Above the kernel: the pools' version counters move, so that a backward that
-// saved a pool before a prompt entered it raises, as after slice copies.
-void write_prefix_versioned(at::Tensor& cache_k, at::Tensor& cache_v, const at::Tensor& k,
-                            const at::Tensor& v, at::IntArrayRef pages) {
+// Above the kernel: pools or rows that autograd tracks, or that carry a tangent,
+// are copied page by page with ops that have derivatives (and refuse a leaf
+// pool).  Otherwise the pools' version counters move, so that a backward that
+// saved a pool before a prompt entered it raises, as after those copies.
+void write_prefix_autograd(at::Tensor& cache_k, at::Tensor& cache_v, const at::Tensor& k,
+                           const at::Tensor& v, at::IntArrayRef pages) {
+  auto tracked = [](const at::Tensor& x) {
+    return (x.requires_grad() && at::GradMode::is_enabled()) || x._fw_grad(0).defined();
+  };
+  if (tracked(cache_k) || tracked(cache_v) || tracked(k) || tracked(v)) {
+    for (size_t i = 0; i < pages.size(); ++i) {
+      if (pages[i] < 0 || pages[i] >= cache_k.size(0)) continue;
+      const int64_t t0 = int64_t(i) * BC_PAGE_SIZE;
+      const int64_t n = std::min<int64_t>(BC_PAGE_SIZE, k.size(0) - t0);
+      cache_k.select(0, pages[i]).narrow(0, 0, n).copy_(k.narrow(0, t0, n));
+      cache_v.select(0, pages[i]).narrow(0, 0, n).copy_(v.narrow(0, t0, n));
+    }
+    return;
+  }
   static const auto op =
       c10::Dispatcher::singleton()
           .findSchemaOrThrow("branchcraft::write_prefix_", "")
@@ -429,6 +444,6 @@ TORCH_LIBRARY_IMPL(branchcraft, CUDA, m) {
   m.impl("paged_decode", paged_decode_hip);
 }
 
-TORCH_LIBRARY_IMPL(branchcraft, ADInplaceOrView, m) {
-  m.impl("write_prefix_", write_prefix_versioned);
+TORCH_LIBRARY_IMPL(branchcraft, Autograd, m) {
+  m.impl("write_prefix_", write_prefix_autograd);
 }

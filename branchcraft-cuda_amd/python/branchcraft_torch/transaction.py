@@ -16,7 +16,6 @@ as committing them one by one in the same order.
 from __future__ import annotations
 
 import torch
-from torch.autograd import forward_ad
 
 from . import (commit_path_, commit_paths_, copy_pages_, int_tensor, tree_verify,
                write_prefix_)
@@ -69,19 +68,15 @@ class PagedTreeCache:
                       prefix_v: torch.Tensor) -> None:
         """Prompt rows into fresh pages: one launch, the page ids in its
         kernel arguments.  What the op does not take -- a pool that is not on
-        the GPU, pools or rows that autograd tracks or that carry a tangent, a
-        subclass, or rows that are views of the pool itself -- is copied page
-        by page."""
+        the GPU, a subclass, or rows that are views of the pool itself -- is
+        copied page by page."""
         rows = [prefix_k, prefix_v]
-        if self.k.is_cuda and all(
-                type(x) in (torch.Tensor, torch.nn.Parameter)
-                and not (x.requires_grad and torch.is_grad_enabled())
-                and forward_ad.unpack_dual(x).tangent is None
-                for x in (self.k, self.v, *rows)):
+        if self.k.is_cuda and {*map(type, (self.k, *rows))} <= {torch.Tensor, torch.nn.Parameter}:
             store = [x.untyped_storage().data_ptr() for x in (self.k, self.v)]
             if not any(x.untyped_storage().data_ptr() in store for x in rows):
                 # V of another type or device is converted as a copy would.
-                rows = [x.to(self.k.device, torch.float16) for x in rows]
+                if prefix_v.dtype != torch.float16 or prefix_v.device != self.k.device:
+                    rows[1] = prefix_v.to(self.k.device, torch.float16)
                 rows = [x if x.stride(-1) == 1 else x.contiguous() for x in rows]
                 if pages:
                     write_prefix_(self.k, self.v, *rows, pages)
