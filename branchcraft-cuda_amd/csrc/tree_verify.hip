@@ -31,11 +31,13 @@
 //    pages run on the same XCD and reuse its L2.
 //  - tree_wide_kernel: trees of several row tiles per (request, KV head): four
 //    waves take four row tiles (or two, two waves each) and share K/V tiles
-//    that are loaded straight into LDS, whole units or shares of them, which
-//    merge_wide_kernel combines.
-//  - tree_flat_kernel: small trees over batches of long prefixes that stream
-//    from HBM: every workgroup takes an equal range of the batch's tiles, and
-//    merge_flat_kernel combines the units that a range boundary cuts.
+//    that are loaded straight into LDS, whole units or shares of them.
+//  - tree_flat_kernel: small trees over batches that may be long and ragged:
+//    every workgroup takes an equal range of the batch's tiles.
+//  - tree_whole_kernel, behind a launch of shares or ranges: the host sees only
+//    what a page table could hold, so those launches read the lengths and leave
+//    a batch that is better off whole to this kernel, which verifies it in a
+//    single pass; else it combines the partials of the units that were cut.
 //  - tree_rows_kernel, tree_kernel: element-wise loads and stores, for tensors
 //    that are not 16-byte aligned (and, tree_kernel, calls without the pool
 //    size): a K/V tile shared by four row tiles, and one row tile each.
@@ -80,8 +82,11 @@ struct TreeParams {
   // tree_split_kernel: parts per unit and tiles per part; with parts > 1,
   // part_acc/part_ml hold P.parts slots per output row.  tree_wide_kernel:
   // workgroups that split the units (1: none are split), with a slot per
-  // workgroup and row of its, and the CUs they run on.
+  // workgroup and row of its.  tree_flat_kernel: ranges.
   int parts, tiles_per_part;
+  // The device's CUs, and the rounds over them of the same units whole
+  // (tree_wide_kernel's shares and tree_flat_kernel).
+  int cus, whole_rounds;
   // ceil(2^32 / d) for d = group and d = row_tiles (0: divide plainly), and
   // whether the launch is a (KV head x row tile, request group, part) grid.
   unsigned long long group_mul, rt_mul;
@@ -98,7 +103,7 @@ __device__ __forceinline__ void pin_params(const TreeParams& P) {
                "s"(P.batch), "s"(P.nodes), "s"(P.hq), "s"(P.hkv), "s"(P.group),
                "s"(P.max_pages), "s"(P.phys_pages), "s"(P.rows), "s"(P.row_tiles),
                "s"(P.scale_log2), "s"(P.parts), "s"(P.tiles_per_part), "s"(P.group_mul),
-               "s"(P.rt_mul), "s"(P.grid3d));
+               "s"(P.rt_mul), "s"(P.grid3d), "s"(P.cus), "s"(P.whole_rounds));
   __builtin_amdgcn_sched_barrier(0);  // nothing that uses them moves above
 }
 
@@ -635,8 +640,10 @@ __device__ __forceinline__ void wave_lds_sync() {
 // workspace) that share goes to the output, otherwise every part with tiles
 // writes an FP32 partial per row, slot (row, part), and merge_split_kernel
 // combines them.
-template <int D, int W, int RQ>
-__global__ __launch_bounds__(64 * W, 2) void tree_split_kernel(TreeParams P) {
+// WHOLE: one part per unit on a flat grid (tree_whole_kernel), whatever the
+// parameters say of parts.
+template <int D, int W, int RQ, bool WHOLE>
+__device__ __forceinline__ void tree_split_body(const TreeParams& P) {
   constexpr int KS = D / 16;      // MFMA k-steps; also load instructions per tile
   constexpr int DT = D / 32;      // 32-row output tiles over the head dimension
   constexpr int KP = D + 8;       // halves per staged K row
@@ -647,7 +654,6 @@ __global__ __launch_bounds__(64 * W, 2) void tree_split_kernel(TreeParams P) {
   constexpr int STAGE = kTile * (KP + VP);  // halves per wave
   constexpr int LN = W / RQ;      // waves per request
 
-  pin_params(P);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 5;   // lane half
@@ -661,15 +667,16 @@ __global__ __launch_bounds__(64 * W, 2) void tree_split_kernel(TreeParams P) {
   // Workgroup ids put (KV head, row tile) in the low bits, then the request
   // group, then the part (a 3-D grid, or the same order flattened).
   int z, b0, part;
-  if (P.grid3d) {
+  if (!WHOLE && P.grid3d) {
     z = blockIdx.x;
     b0 = blockIdx.y * RQ;
     part = blockIdx.z;
   } else {
     const int zdim = P.hkv * P.row_tiles;
     const int units = zdim * ((P.batch + RQ - 1) / RQ);
-    const int unit = blockIdx.x % units;
-    part = blockIdx.x / units;
+    const int unit = WHOLE ? blockIdx.x : blockIdx.x % units;
+    part = WHOLE ? 0 : blockIdx.x / units;
+    if (WHOLE && unit >= units) return;  // uniform: the grid has a workgroup per CU at least
     z = unit % zdim;
     b0 = (unit / zdim) * RQ;
   }
@@ -677,7 +684,7 @@ __global__ __launch_bounds__(64 * W, 2) void tree_split_kernel(TreeParams P) {
   const int b = present ? b0 + rq : b0;    // absent waves read request b0, unused
   const int kvh = div_by(z, P.row_tiles, P.rt_mul);
   const int rt = z - kvh * P.row_tiles;
-  const int T = P.tiles_per_part;
+  const int T = WHOLE ? 1 << 30 : P.tiles_per_part;
   const int tbeg = part * T;
 
   // Page ids of this wave's tiles as vector loads (lane j: page j%2 of the
@@ -1091,7 +1098,7 @@ __global__ __launch_bounds__(64 * W, 2) void tree_split_kernel(TreeParams P) {
   const int rrn = div_by(rr, P.group, P.group_mul);
   const size_t orow =
       ((size_t)b * P.nodes + rrn) * P.hq + kvh * P.group + (rr - rrn * P.group);
-  if (P.parts == 1) {
+  if (WHOLE || P.parts == 1) {
     const float inv = 1.f / ll;  // every row sees its own node: ll > 0
     float* dst = P.out + orow * D + md0;
 #pragma unroll
@@ -1106,6 +1113,12 @@ __global__ __launch_bounds__(64 * W, 2) void tree_split_kernel(TreeParams P) {
       *reinterpret_cast<float4*>(dst + j) = make_float4(o[j], o[j + 1], o[j + 2], o[j + 3]);
     if (md0 == 0) *reinterpret_cast<float2*>(P.part_ml + 2 * slot) = make_float2(mm, ll);
   }
+}
+
+template <int D, int W, int RQ>
+__global__ __launch_bounds__(64 * W, 2) void tree_split_kernel(TreeParams P) {
+  pin_params(P);
+  tree_split_body<D, W, RQ, false>(P);
 }
 
 // Combines tree_split_kernel's partials: one wave per output row (b, node,
@@ -1303,14 +1316,53 @@ __device__ __forceinline__ int2* wide_records(const TreeParams& P) {
   return reinterpret_cast<int2*>(P.part_ml + (size_t)P.parts * RT * 32 * 2);
 }
 
+// Set by the split launch for tree_whole_kernel behind it: whether the shares
+// were taken, and not left to that kernel as whole units.
+template <int RT>
+__device__ __forceinline__ int* wide_taken(const TreeParams& P) {
+  return reinterpret_cast<int*>(wide_records<RT>(P) + P.batch);
+}
+
+// The tiles that one CU takes one after the other where a single pass runs
+// whole units (tree_whole_kernel), as far as the lengths tell: `all` tiles of
+// the requests together, `longest` of the longest.  Each round over the CUs
+// ends with its longest unit at the latest, and no CU gets more than its equal
+// part and a unit.
+__device__ __forceinline__ float whole_chain(const TreeParams& P, int all, int longest) {
+  return __builtin_fminf((float)P.whole_rounds * (float)longest,
+                         (float)all * (float)(P.hkv * P.row_tiles) / (float)P.cus + (float)longest);
+}
+
+// Whether shares of the batch's units beat whole ones.  Shares take a CU's part
+// of the row groups, and finding, leaving and merging them costs the time of 56
+// tiles (15 us); 44 where the tiles, each read once per row tile by whole units,
+// are more than the L2s hold.  With two units per CU (D = 64: more) shares win
+// at any length.  Over 119 batches of 1 to 64 requests x 33 to 8192 tokens,
+// under tables of up to 32768, the rule takes 0.1 % longer than the faster of
+// both on average and 5 % at most.  Shares against whole units, us, 32/8 heads
+// and D = 128 unless noted: 1 x 300 x 256 nodes 28 against 17, 16 x 64-512 x 16
+// 20 against 17, 5 x 2102 x 33 (32/4, one shared prefix) 35 against 27, 16 x
+// 2454 x 16 (24/8, D = 64, shared) 25 against 22, 16 x 64-512 x 33 (28/4, D =
+// 64) 19 against 16; 2 x 1058-2117 x 9 19 against 24, 14 x 2319 x 32 54 against
+// 90, 16 x 200-900 x 64 39 against 62, 16 x 300-3000 x 33 (28/4, D = 64) 31
+// against 47.
+template <int D>
+__device__ __forceinline__ bool wide_pays(const TreeParams& P, int all, int longest, int zdim) {
+  const float cus = (float)P.cus;
+  const float units = (float)P.batch * (float)(P.hkv * P.row_tiles);
+  const bool far = (float)all * (float)(kTile * 4 * D) * (float)P.hkv > 32e6f;
+  return units >= 2.f * cus + (D == 64 ? 1.f : 0.f) ||
+         whole_chain(P, all, longest) > (float)all * (float)zdim / cus + (far ? 44.f : 56.f);
+}
+
 // Workgroup blockIdx.x's share when P.parts workgroups split the units on
-// P.tiles_per_part CUs: the shortest share of at least kWideLeast steps with
+// P.cus CUs: the shortest share of at least kWideLeast steps with
 // which the batch, however ragged, needs no more than P.parts workgroups,
 // from the lengths themselves (parts == 0: none left).  A request's units
 // take equal shares.
 // Every wave finds it for itself, a lane holding four requests; counts of a
 // share per lane add up by ballots of their six bits.
-template <int RT>
+template <int D, int RT>
 __device__ __forceinline__ WidePart wide_part(const TreeParams& P, int lane, int zdim) {
   constexpr int NW = kWideRequests / 64;
   int len[NW], steps[NW], sum = 0, most = 0;
@@ -1327,6 +1379,9 @@ __device__ __forceinline__ WidePart wide_part(const TreeParams& P, int lane, int
   // Uniform values in scalar registers keep the search scalar.
   const int all = __builtin_amdgcn_readfirstlane(wave_sum_i(sum));
   const int longest = __builtin_amdgcn_readfirstlane((int)wave_max((float)most));
+  const bool taken = wide_pays<D>(P, 2 * all, 2 * longest, zdim);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *wide_taken<RT>(P) = taken;
+  if (!taken) return WidePart{0, 0, 0, 0, 0, 0};
   const int cap = P.parts / zdim;  // shares of all requests, >= P.batch
   // About ceil(steps / per): 1 to kWideParts, no more than steps, and 1 for
   // per == longest.  Shares follow from the count, so that it need not be exact.
@@ -1343,7 +1398,7 @@ __device__ __forceinline__ WidePart wide_part(const TreeParams& P, int lane, int
   // 3696 x 11 (28/4 heads) 129 against 114, 8 x 8000 x 128 217 against 206, 28
   // x 6000 x 48 (16/4, D = 64) 111 against 94, 16 x 4096 x 64 (D = 64) 83
   // against 79.
-  if (1.2f * (float)longest <= (float)all * (float)zdim / (float)P.tiles_per_part + kWideSlack)
+  if (1.2f * (float)longest <= (float)all * (float)zdim / (float)P.cus + kWideSlack)
     per = max(per, longest);
   for (int hi = max(per, longest); per < hi;) {
     const int mid = (per + hi) >> 1;
@@ -1402,7 +1457,7 @@ __device__ __forceinline__ WidePart wide_part(const TreeParams& P, int lane, int
 // computed, one barrier per step, and hold no registers, so the reads of a
 // whole step's K can be in flight at once.  A whole unit's rows go to the
 // output, a share leaves an FP32 partial of each row, in the workgroup's own
-// slots, for merge_wide_kernel.
+// slots, for merge_wide.
 // Bound by the matrix units and their clock: 8 requests x 2048 tokens x 256
 // nodes (32/8 heads, D = 128) take 112 us, 617 TFLOP/s (925 with the second
 // MFMA that P's low part takes); the MFMAs alone fill half the cycles, and
@@ -1441,7 +1496,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
   const int zdim = P.hkv * rgroups;
   WidePart w{0, 0, 0, 0, 0, 1};
   if constexpr (SPLIT) {
-    w = wide_part<RT>(P, lane, zdim);
+    w = wide_part<D, RT>(P, lane, zdim);
     if (w.parts == 0) return;  // uniform
   } else {
     w.b = blockIdx.x / zdim;
@@ -1453,7 +1508,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
   // Whole units: the later row groups of a tree see more of its draft tiles
   // (below), so every other round of workgroups over the CUs takes them in the
   // opposite order.
-  if (!SPLIT && ((b * P.hkv + kvh) * rgroups / P.tiles_per_part) & 1) rg = rgroups - 1 - rg;
+  if (!SPLIT && ((b * P.hkv + kvh) * rgroups / P.cus) & 1) rg = rgroups - 1 - rg;
 
   // First round of loads: the page ids (lane i of a register: entry i of the
   // 64 table entries from step t on, from inside the request's table row),
@@ -1855,62 +1910,95 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void tree_wide_kernel(TreePar
 }
 
 // Combines the partials of the units that a split launch of tree_wide_kernel
-// cut: one wave per output row (b, node, h).  Lane p holds share p's (max,
-// sum); the weights are formed once and every lane accumulates its dims from
-// the shares, eight at a time.
-template <int D, int RT>
-__global__ __launch_bounds__(256) void merge_wide_kernel(TreeParams P) {
-  pin_params(P);
-  constexpr int PER = D / 64;
+// cut: wave `worker` of `workers` takes every workers-th group of CH rows of a
+// unit, D / 4 lanes on a row, so that the count of shares is the wave's own and
+// the rows' loads of a round, U shares of each, are in flight together.
+template <int RT, int CH>
+__device__ __forceinline__ int2 merge_wide_record(const TreeParams& P, int item) {
+  const int zdim = P.hkv * ((P.row_tiles + RT - 1) / RT);
+  constexpr int chunks = RT * 32 / CH;
+  return wide_records<RT>(P)[min(item / chunks / zdim, P.batch - 1)];
+}
+
+template <int D, int RT, int CH, int U>
+__device__ __forceinline__ void merge_wide(const TreeParams& P, int worker, int workers,
+                                           int2 rec_next) {
+  constexpr int C4 = D / 4;      // lanes per row, four dims each
+  constexpr int RPW = 64 / C4;   // rows side by side in a wave
+  constexpr int R = CH / RPW;
+  constexpr int chunks = RT * 32 / CH;
   const int lane = threadIdx.x & 63;
-  const unsigned row =
-      __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));  // (b*N+node)*Hq+h
-  if (row >= (unsigned)P.batch * P.nodes * P.hq) return;
-  const unsigned bn = row / P.hq, h = row - bn * P.hq;
-  const unsigned b = bn / P.nodes, node = bn - b * P.nodes;
-  const int2 rec = wide_records<RT>(P)[b];
-  const int parts = __builtin_amdgcn_readfirstlane(rec.y);
-  if (parts < 2) return;  // written by its only share
-  const int kvh = h / P.group, r = node * P.group + (h - kvh * P.group);
+  const int sub = lane / C4, c = 4 * (lane % C4);
   const int rgroups = (P.row_tiles + RT - 1) / RT, zdim = P.hkv * rgroups;
-  const int rg = r / (RT * 32);
-  const size_t slot0 =
-      ((size_t)__builtin_amdgcn_readfirstlane(rec.x) * zdim + kvh * rgroups + rg) * (RT * 32) +
-      (r - rg * (RT * 32));
+  const int items = P.batch * zdim * chunks;
   const size_t next = (size_t)zdim * (RT * 32);  // from a share's slot to the next one's
-  const float2 ml =
-      *reinterpret_cast<const float2*>(P.part_ml + 2 * (slot0 + min(lane, parts - 1) * next));
-  float x[8][PER], a[PER];
-  auto load = [&](int p0) {
+  for (int item = worker; item < items; item += workers) {
+    const int2 rec = rec_next;
+    rec_next = merge_wide_record<RT, CH>(P, item + workers);
+    const int unit = item / chunks, ch = item % chunks;
+    const int b = unit / zdim, z = unit - b * zdim;
+    const int kvh = z / rgroups, rg = z - kvh * rgroups;
+    const int r0 = rg * (RT * 32) + ch * CH;
+    const int parts = __builtin_amdgcn_readfirstlane(rec.y);
+    if (r0 >= P.rows || parts < 2) continue;  // no rows, or written by its only share
+    const size_t slot0 =
+        ((size_t)__builtin_amdgcn_readfirstlane(rec.x) * zdim + z) * (RT * 32) + ch * CH + sub;
+    float m[R], l[R];
+    float4 a[R];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const float* src = P.part_acc + (slot0 + min(p0 + u, parts - 1) * next) * D + lane;
-#pragma unroll
-      for (int j = 0; j < PER; ++j) x[u][j] = src[64 * j];
+    for (int i = 0; i < R; ++i) {
+      m[i] = kNegInf;
+      l[i] = 0.f;
+      a[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-  };
-  load(0);
-  const float mp = lane < parts ? ml.x : kNegInf;
-  // Every share holds the row's partial; one of them has its own node, so
-  // the max is finite.
-  const float w = fast_exp2(mp - wave_max(mp));
-  const float lsum = wave_sum(lane < parts ? w * ml.y : 0.f);
+    for (int p0 = 0; p0 < parts; p0 += U) {
+      float2 ml[U][R];
+      float4 v[U][R];
 #pragma unroll
-  for (int j = 0; j < PER; ++j) a[j] = 0.f;
-  for (int p0 = 0; p0 < parts; p0 += 8) {
-    if (p0 > 0) load(p0);
+      for (int u = 0; u < U; ++u) {
+        const size_t at = slot0 + min(p0 + u, parts - 1) * next;
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (p0 + u < parts) {  // uniform
-        const float wi = __builtin_bit_cast(
-            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), p0 + u));
-#pragma unroll
-        for (int j = 0; j < PER; ++j) a[j] += wi * x[u][j];
+        for (int i = 0; i < R; ++i) {
+          ml[u][i] = *reinterpret_cast<const float2*>(P.part_ml + 2 * (at + i * RPW));
+          v[u][i] = *reinterpret_cast<const float4*>(P.part_acc + (at + i * RPW) * D + c);
+        }
       }
-  }
-  const float inv = 1.f / lsum;
 #pragma unroll
-  for (int j = 0; j < PER; ++j) P.out[(size_t)row * D + lane + 64 * j] = a[j] * inv;
+      for (int i = 0; i < R; ++i) {
+        float mn = m[i];
+#pragma unroll
+        for (int u = 0; u < U; ++u) mn = __builtin_fmaxf(mn, ml[u][i].x);  // the last one again
+        const float ms = safe_max(mn);
+        const float keep = fast_exp2(m[i] - ms);
+        l[i] *= keep;
+        a[i].x *= keep;
+        a[i].y *= keep;
+        a[i].z *= keep;
+        a[i].w *= keep;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const float w = p0 + u < parts ? fast_exp2(ml[u][i].x - ms) : 0.f;
+          l[i] += w * ml[u][i].y;
+          a[i].x += w * v[u][i].x;
+          a[i].y += w * v[u][i].y;
+          a[i].z += w * v[u][i].z;
+          a[i].w += w * v[u][i].w;
+        }
+        m[i] = mn;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int r = r0 + sub + i * RPW;
+      if (r < P.rows) {
+        const int node = div_by(r, P.group, P.group_mul);
+        const float inv = 1.f / l[i];  // every row sees its own node
+        *reinterpret_cast<float4*>(
+            P.out + (((size_t)b * P.nodes + node) * P.hq + kvh * P.group + (r - node * P.group)) * D +
+            c) = make_float4(a[i].x * inv, a[i].y * inv, a[i].z * inv, a[i].w * inv);
+      }
+    }
+  }
 }
 
 // ---- flat ranges: equal shares of a ragged batch's tiles ----
@@ -1945,6 +2033,30 @@ struct FlatPos {
   int ord, z, b, len, t, tend, rest;
 };
 
+// What merge_flat_range needs of each range, after the partials' (max, sum)
+// pairs (two slots of 32 rows per range): the unit it begins in and how many
+// tiles into it (an empty range: unit -1, tile 0).
+__device__ __forceinline__ int2* flat_records(const TreeParams& P) {
+  return reinterpret_cast<int2*>(P.part_ml + (size_t)P.parts * 2 * 32 * 2);
+}
+
+// As wide_taken.
+__device__ __forceinline__ int* flat_taken(const TreeParams& P) {
+  return reinterpret_cast<int*>(flat_records(P) + P.parts);
+}
+
+// Whether equal ranges beat whole units: where the longest chain of a single
+// pass exceeds an equal part by the time that ranges cost, 48 tiles.  Over 118
+// batches as at wide_pays 0.3 % longer than the faster of both on average, 11 %
+// at most.  Ranges against whole units, us, 7 nodes, 32/8 heads and D = 128
+// unless noted: 64 x 16-200 29 against 16, 64 x 32-1024 46 against 42, 64 x 2048
+// (one shared prefix) 54 against 49, 32 x 64-2048 45 against 41; 64 x 128-4096
+// 115 against 134 (D = 64: 67 against 77), 16 x 128-4096 47 against 60, 4 x
+// 500-8000 x 8 nodes 30 against 74.
+__device__ __forceinline__ bool flat_pays(const TreeParams& P, int all, int longest, int zdim) {
+  return whole_chain(P, all, longest) > (float)all * (float)zdim / (float)P.cus + 48.f;
+}
+
 // Range rid's first position (ord -1: the range is empty), of P.parts equal
 // ranges.  Units are ordered z (KV head, row tile) outermost, then request:
 // a range of one KV head's tiles finds requests that share pages next to
@@ -1952,18 +2064,22 @@ struct FlatPos {
 __device__ __forceinline__ FlatPos flat_first(const TreeParams& P, int lane, int rid, int zdim,
                                               FlatLens& lens) {
   const int len0 = flat_len(P, min(lane, P.batch - 1));
-  int s = lane < P.batch ? flat_tiles(P, len0) : 0;
+  int sum = lane < P.batch ? flat_tiles(P, len0) : 0, most = sum;
   for (int base = 64; base < P.batch; base += 64) {
     const int i = base + lane;
-    s += i < P.batch ? flat_tiles(P, flat_len(P, min(i, P.batch - 1))) : 0;
+    const int n = i < P.batch ? flat_tiles(P, flat_len(P, min(i, P.batch - 1))) : 0;
+    sum += n;
+    most = max(most, n);
   }
-  // The sum is the same in every lane; in a scalar register it keeps the
-  // whole walk scalar.
-  const int all = __builtin_amdgcn_readfirstlane(wave_sum_i(s));
+  // Sums in scalar registers keep the whole walk scalar.
+  const int all = __builtin_amdgcn_readfirstlane(wave_sum_i(sum));
+  const int longest = __builtin_amdgcn_readfirstlane((int)wave_max((float)most));
+  const bool taken = flat_pays(P, all, longest, zdim);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *flat_taken(P) = taken;
   const int total = all * zdim;
   const int per = (total + P.parts - 1) / P.parts;
   const int f0 = rid * per;
-  const int count = min(total - f0, per);
+  const int count = taken ? min(total - f0, per) : 0;
   FlatPos p{-1, 0, 0, 0, 0, 0, 0};
   lens = FlatLens{0, len0};
   if (count <= 0) return p;
@@ -2012,13 +2128,6 @@ __device__ __forceinline__ int flat_range_id(const TreeParams& P) {
   return n % 8 == 0 ? i % 8 * (n / 8) + i / 8 : i;
 }
 
-// What merge_flat_kernel needs of each range, after the partials' (max, sum)
-// pairs (two slots of 32 rows per range): the unit it begins in and how many
-// tiles into it (an empty range: unit -1, tile 0).
-__device__ __forceinline__ int2* flat_records(const TreeParams& P) {
-  return reinterpret_cast<int2*>(P.part_ml + (size_t)P.parts * 2 * 32 * 2);
-}
-
 __device__ __forceinline__ void flat_record(const TreeParams& P, int rid, const FlatPos& p) {
   if (threadIdx.x == 0)
     flat_records(P)[rid] = p.ord < 0 ? make_int2(-1, 0) : make_int2(p.z * P.batch + p.b, p.t);
@@ -2033,7 +2142,7 @@ __device__ __forceinline__ void flat_record(const TreeParams& P, int rid, const 
 // with its own staging area and no barrier; at the segment's end they merge
 // through LDS.  A unit that lies inside one range is written directly; the
 // others leave one FP32 partial per range (slot 2r for the range's first
-// segment, 2r + 1 for its last), which merge_flat_kernel combines.
+// segment, 2r + 1 for its last), which merge_flat_range combines.
 // Bound by HBM: a wave requests its next tile, also across a segment's end,
 // before it computes the current one, with non-temporal loads (plain ones: 13
 // us more at the shape below), ahead of the waves that compute.  64 requests x
@@ -2338,21 +2447,18 @@ __global__ __launch_bounds__(64 * W, 2) void tree_flat_kernel(TreeParams P) {
   }
 }
 
-// Combines tree_flat_kernel's partials: one workgroup per range boundary r.
-// The unit that
-// range r starts inside is merged at the first boundary that cuts it, over
+// Combines tree_flat_kernel's partials at range boundary r, 256 threads on it.
+// The unit that range r starts inside is merged at the first boundary that cuts it, over
 // range r - 1 and the ranges from r on that start inside it too; every other
 // unit lies inside one range and was written by the attention kernel.  Range
 // r - 1 holds the unit as its first segment (slot 2(r - 1)) or, when the
 // unit begins inside it, its last (slot 2(r - 1) + 1); the others as their
 // first.
 template <int D>
-__global__ __launch_bounds__(256) void merge_flat_kernel(TreeParams P) {
-  pin_params(P);
+__device__ __forceinline__ void merge_flat_range(const TreeParams& P, int r) {
   constexpr int NF = D / 32;  // float4s per thread: 8 threads per row
   constexpr int U = 4;        // parts loaded together
   const int lane = threadIdx.x & 63;
-  const int r = 1 + blockIdx.x;
   const int2* rec = flat_records(P);
   const int2 m1 = rec[r], m0 = rec[r - 1];
   const int mv = rec[min(r + 1 + lane, P.parts - 1)].x;
@@ -2369,7 +2475,7 @@ __global__ __launch_bounds__(256) void merge_flat_kernel(TreeParams P) {
     nparts += n;
     if (n < 64 || base + 64 >= P.parts) break;
   }
-  const int row = threadIdx.x >> 3, d0 = 4 * (threadIdx.x & 7);
+  const int row = threadIdx.x % 256 >> 3, d0 = 4 * (threadIdx.x & 7);
   const int z = unit / P.batch, b = unit - z * P.batch;
   const int kvh = div_by(z, P.row_tiles, P.rt_mul);
   const int rr = (z - kvh * P.row_tiles) * 32 + row;
@@ -2427,6 +2533,36 @@ __global__ __launch_bounds__(256) void merge_flat_kernel(TreeParams P) {
   for (int j = 0; j < NF; ++j)
     *reinterpret_cast<float4*>(dst + 32 * j) =
         make_float4(a[j].x * inv, a[j].y * inv, a[j].z * inv, a[j].w * inv);
+}
+
+// Behind a launch that cut a batch's units by its lengths, or found that whole
+// units serve it better (RT: row tiles a workgroup of tree_wide_kernel, 0:
+// tree_flat_kernel): combines the partials, or verifies the whole units as
+// tree_split_kernel does in a single pass.  One launch for both, as an empty one
+// costs 1.5 us; its grid has a workgroup per CU at least.
+template <int D, int RQ, int RT>
+__global__ __launch_bounds__(512, 2) void tree_whole_kernel(TreeParams P) {
+  pin_params(P);
+  if constexpr (RT > 0) {
+    // Eight rows a wave, or four where the units are few and so in many shares
+    // each (22 x 1934 x 9 nodes, 16/2 heads, D = 128: 31.8 -> 29.0 us).  The
+    // first record is loaded with the word that says whether there are any.
+    const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 8 + (threadIdx.x >> 6));
+    const int waves = P.cus * 8;  // of a workgroup per CU
+    const bool few = P.batch * P.hkv * ((P.row_tiles + RT - 1) / RT) * (RT * 8) <= waves;
+    const int taken = *wide_taken<RT>(P);
+    int2 rec = few ? merge_wide_record<RT, 4>(P, wave) : merge_wide_record<RT, 8>(P, wave);
+    asm volatile("" : "+v"(rec.x), "+v"(rec.y));
+    if (!taken) tree_split_body<D, 8, RQ, true>(P);
+    else if (wave >= waves) return;
+    else if (few) merge_wide<D, RT, 4, 8>(P, wave, waves, rec);
+    else merge_wide<D, RT, 8, 4>(P, wave, waves, rec);
+  } else if (!*flat_taken(P)) {
+    tree_split_body<D, 8, RQ, true>(P);
+  } else {
+    const int r = 1 + blockIdx.x * 2 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    if (r < P.parts) merge_flat_range<D>(P, r);  // a workgroup per CU and so per range
+  }
 }
 
 // Row-sharing variant, for tensors that are not 16-byte aligned, of trees of
@@ -2745,6 +2881,7 @@ TreeParams make_params(const bc_shape& s, const bc_tree_inputs& in, int nodes) {
   // (bindings/torch_ops.cpp:54 passes prefix_k.size(0)); below 1 the ids
   // are not range-checked (tree_kernel only, see pool_known).
   P.phys_pages = pool_known(s) ? s.physical_pages : 0x7fffffff;
+  P.cus = bch::device_cus();
   P.rows = nodes * P.group;
   P.row_tiles = (P.rows + 31) / 32;
   P.scale_log2 = (float)(1.4426950408889634 / __builtin_sqrt((double)s.dim));
@@ -2785,7 +2922,7 @@ bool tree_ptrs_aligned(const bc_tree_inputs& in) {
 
 struct SplitPlan {
   int parts;  // workgroups per (request group, KV head, row tile), <= 64
-  int tiles;  // 32-token tiles per workgroup and request (draft then prefix tiles); wide: CUs
+  int tiles;  // 32-token tiles per workgroup and request (draft then prefix tiles)
   int waves;  // waves per workgroup: 4 or 8
   int rq = 1;  // requests per workgroup (waves / rq per request)
   int wide = 0;  // row tiles per workgroup of tree_wide_kernel (0: tree_split_kernel)
@@ -2800,25 +2937,21 @@ long long row_groups(const bc_shape& s, int row_tiles, int rt) {
 // tree_split_kernel reads it per row tile, so it takes the trees of several
 // row tiles whose groups fill the CUs (same box, 32/8 heads and D = 128 unless
 // noted, tree_split_kernel or the kernel it replaced first):
-//  - long prefixes (60 tiles), at most one group per CU, and at least 17 steps
-//    per CU in all (D = 64, whose steps are half as long: 24): two workgroups
-//    per CU split the groups by the batch's lengths, four row tiles each (two,
-//    if there are no more).  Against equal parts of the table's capacity: 8 x
-//    128-4096 tokens x 128 nodes 110 -> 67 us, 4 x 500-8000 x 128 88 -> 55, 32
-//    x 256-2048 x 16 48 -> 43, 28/4 heads, D = 64: 16 x 300-3000 x 33 35 ->
-//    31; equal lengths pay 2 to 4 us for finding the share and for the merge
-//    launch: 8 x 2048 x 128 65 -> 69 (103 by tree_split_kernel).  Less work leaves each share too few steps to pay
-//    for its partial rows (16/2 heads: 4 x 4000 x 128 nodes 42 against 46 us,
-//    8 x 2048 x 64 25 against 35; 28/4 heads, D = 64: 28 against 34);
-//    but prefixes of more than 32 MB, which the eight L2s do not hold, cost
-//    tree_split_kernel a trip past the L2 per row tile, and from 5 steps per CU
-//    (D = 64: 12) the shares win: 14 x 2319 x 32 nodes 86 against 47 us, 9 x
-//    450-3600 x 32 (32/4) 74 against 38, 6 x 1079-2158 x 12 (24/8) 22.3 against
-//    19.3, 22 x 1934 x 9 (16/2) 28.5 against 27.2, D = 64: 21 x 2333 x 16 (28/4)
-//    36 against 27; fewer steps: 10 x 1041-2082 x 20 (D = 64) 22.0 against 24.3.
-//    On prefixes that do not reach it, shared by the requests or few, the rule
-//    above stays: 16 x 2454 x 16 (24/8, D = 64, one shared prefix) 18 against
-//    23, 5 x 2102 x 33 (32/4, shared) 22 against 32;
+//  - tables of 60 tiles and more, at most one group per CU, and room for at
+//    least 17 steps per CU in all (D = 64, whose steps are half as long: 24), or
+//    from 5 (D = 64: 12) where tables and pool have room for more than 32 MB,
+//    which the eight L2s do not hold: two workgroups per CU split the groups by
+//    the batch's lengths, four row tiles each (two, if there are no more), if
+//    the lengths fill what the table has room for (wide_pays), else
+//    tree_whole_kernel runs a single pass of whole units.  Below these lines no
+//    lengths make the shares pay, and the second launch (2 us) is saved.  At
+//    lengths that fill the table: 8 x 128-4096 tokens x 128 nodes 185 against
+//    105 us, 14 x 2319 x 32 88 against 47, 9 x 450-3600 x 32 (32/4) 73 against
+//    41, 32 x 256-2048 x 16 58 against 42, 16 x 300-3000 x 33 (28/4, D = 64) 45
+//    against 31, 8 x 2048 x 128 108 against 80; near the lines 22 x 1934 x 9
+//    (16/2) 29.5 against 29.3, 6 x 1079-2158 x 12 (24/8) 21.5 against 19.9.
+//    Short lengths under a table of 4096: 8 x 100-300 x 33 15.7 against 17.8 (21
+//    in shares), 16 x 64-512 x 16 14.6 against 17.1 (20.6);
 //  - else four row tiles a workgroup from 7/8 CUs of groups on: 8 requests x
 //    2048 tokens x 256 nodes 143 against 116 us, 16 x 1000 x 64 nodes 57
 //    against 40, 64 x 30-500 x 64 nodes 73 against 64;
@@ -2841,12 +2974,10 @@ SplitPlan wide_plan(const bc_shape& s, int row_tiles, int max_tiles, int cus, bo
   if (scratch && max_tiles >= 60 && s.batch <= kWideRequests && g <= cus &&
       g * max_tiles >= least * cus) {
     p.parts = 2 * cus;
-    p.tiles = cus;
     p.wide = rt;
     return p;
   }
   p.parts = 1;
-  p.tiles = cus;
   p.wide = 4;
   if (rt == 4 && 8 * g >= 7LL * cus) return p;
   const long long u = row_groups(s, row_tiles, 2);
@@ -2873,6 +3004,15 @@ SplitPlan pair_requests(int batch, long long units, SplitPlan p, int cus) {
   const long long rounds2 = ((batch + 1) / 2 * per_request + cus - 1) / cus;
   if (2 * rounds2 <= rounds1) p.rq = 2;
   return p;
+}
+
+// Sets the rounds of a single pass and returns its requests per workgroup.
+int whole_requests(TreeParams& P) {
+  const long long units = (long long)P.batch * P.hkv * P.row_tiles;
+  const int rq = pair_requests(P.batch, units, SplitPlan{1, 0, 8}, P.cus).rq;
+  const long long wgs = (long long)((P.batch + rq - 1) / rq) * P.hkv * P.row_tiles;
+  P.whole_rounds = rq * (int)((wgs + P.cus - 1) / P.cus);
+  return rq;
 }
 
 // Parts per unit and tiles per part for `cus` compute units, sized from the
@@ -2936,7 +3076,7 @@ size_t split_workspace(const bc_shape& s, int nodes, const SplitPlan& plan, size
   const size_t slots = plan.wide ? (size_t)plan.parts * plan.wide * 32
                                  : (size_t)s.batch * nodes * s.query_heads * plan.parts;
   *acc_bytes = (slots * s.dim * sizeof(float) + 255) & ~(size_t)255;
-  return *acc_bytes + slots * 2 * sizeof(float) + (plan.wide ? s.batch * sizeof(int2) : 0);
+  return *acc_bytes + slots * 2 * sizeof(float) + (plan.wide ? s.batch * sizeof(int2) + sizeof(int) : 0);
 }
 
 template <int D>
@@ -2950,20 +3090,29 @@ void launch_split_kernel(const TreeParams& P, const SplitPlan& plan, dim3 grid,
     tree_split_kernel<D, 8, 1><<<grid, 512, 0, st>>>(P);
 }
 
+// tree_whole_kernel, `rq` requests a workgroup where it runs whole units.
 template <int D, int RT>
-void launch_wide_kernel(const TreeParams& P, hipStream_t st) {
+void launch_whole_kernel(const TreeParams& P, int rq, hipStream_t st) {
+  const size_t units = (size_t)((P.batch + rq - 1) / rq) * P.hkv * P.row_tiles;
+  const dim3 grid((unsigned)std::max<size_t>(units, P.cus));
+  if (rq == 2) tree_whole_kernel<D, 2, RT><<<grid, 512, 0, st>>>(P);
+  else tree_whole_kernel<D, 1, RT><<<grid, 512, 0, st>>>(P);
+}
+
+template <int D, int RT>
+void launch_wide_kernel(TreeParams& P, hipStream_t st) {
   const size_t groups = (size_t)P.batch * P.hkv * ((P.row_tiles + RT - 1) / RT);
   if (P.parts == 1) {
     tree_wide_kernel<D, RT, false><<<dim3((unsigned)groups), 256, 0, st>>>(P);
     return;
   }
+  const int rq = whole_requests(P);
   tree_wide_kernel<D, RT, true><<<dim3((unsigned)P.parts), 256, 0, st>>>(P);
-  const size_t rows = (size_t)P.batch * P.nodes * P.hq;
-  merge_wide_kernel<D, RT><<<dim3((unsigned)((rows + 3) / 4)), 256, 0, st>>>(P);
+  launch_whole_kernel<D, RT>(P, rq, st);
 }
 
 template <int D>
-hipError_t launch_wide(const TreeParams& P, int row_tiles, hipStream_t st) {
+hipError_t launch_wide(TreeParams& P, int row_tiles, hipStream_t st) {
   if (row_tiles == 2) launch_wide_kernel<D, 2>(P, st);
   else launch_wide_kernel<D, 4>(P, st);
   return hipGetLastError();
@@ -2998,16 +3147,20 @@ hipError_t launch_split(TreeParams& P, int dim, const SplitPlan& plan, void* wor
 // ---- tree_flat_kernel: ranges, workspace and launch ----
 
 // Ranges of tree_flat_kernel (0: not taken): one eight-wave workgroup per CU
-// for batches that stream their prefixes from HBM.  The lengths are on the
-// device, so the shape decides: small trees (one row tile), page tables of at
+// for batches that may be long enough to stream their prefixes from HBM, by
+// what the shape has room for: small trees (one row tile), page tables of at
 // least 2048 tokens that could hold 400 MB, and a pool of at least 128 MB (a
-// smaller one stays in the 256 MB cache, where equal shares gain nothing:
-// requests that share their pages).  Same box, 7 nodes, tree_split_kernel
-// first: 64 x 128-4096 tokens 126 against 105 us, 24 x 128-4096 57 against 42,
-// 20 x 256-8192 87 against 62, 64 x 4096 equal lengths 195 against 190, 64 x
-// 128-4096 at D = 64 73 against 58; below the lines it loses: 64 x 32-1024
-// 32 against 44, 32 x 64-2048 28 against 38, 16 x 128-4096 28 against 33, 32 x
-// 2048 on shared pages 22 against 25 us.
+// smaller one stays in the 256 MB cache, where equal shares gain nothing).  The
+// kernel reads the lengths (flat_pays), and tree_whole_kernel takes what is
+// better off whole.  7 nodes, 32/8 heads, D = 128 unless noted,
+// tree_split_kernel first: 64 x 128-4096 tokens 130 against 115 us, 20 x
+// 256-8192 99 against 84, 64 x 128-4096 at D = 64 73 against 67; under a table
+// of 32768 tokens 16 x 128-4096 62 against 47, 4 x 500-8000 x 8 nodes 51
+// against 30.  Left whole, the second launch and the lengths ahead of the first
+// load cost 2 to 3 us: 64 x 32-1024 39 against 42, 64 x 2048 (one shared prefix)
+// 46 against 49, 64 x 16-200 13 against 16 (in ranges 46, 54 and 29).  Below
+// the lines ranges lose at any length: 64 x 32-1024 32 against 44, 16 x 128-4096
+// 28 against 33.
 int flat_ranges(const bc_shape& s, int nodes, int cus) {
   const int group = s.query_heads / s.kv_heads;
   const long long page = 2LL * BC_PAGE_SIZE * s.kv_heads * s.dim * sizeof(uint16_t);
@@ -3022,13 +3175,14 @@ int flat_ranges(const bc_shape& s, int nodes, int cus) {
 size_t flat_workspace(const bc_shape& s, int ranges, size_t* acc_bytes) {
   const size_t slots = (size_t)2 * ranges * 32;
   *acc_bytes = slots * s.dim * sizeof(float);
-  return *acc_bytes + slots * 2 * sizeof(float) + (size_t)ranges * sizeof(int2);
+  return *acc_bytes + slots * 2 * sizeof(float) + (size_t)ranges * sizeof(int2) + sizeof(int);
 }
 
 template <int D>
-void launch_flat_kernel(const TreeParams& P, hipStream_t st) {
+void launch_flat_kernel(TreeParams& P, hipStream_t st) {
+  const int rq = whole_requests(P);
   tree_flat_kernel<D, 8><<<dim3(P.parts), 512, 0, st>>>(P);
-  if (P.parts > 1) merge_flat_kernel<D><<<dim3(P.parts - 1), 256, 0, st>>>(P);
+  launch_whole_kernel<D, 0>(P, rq, st);
 }
 
 hipError_t launch_flat(TreeParams& P, int dim, int ranges, void* workspace, size_t acc_bytes,
@@ -3079,7 +3233,7 @@ int tree_call(bc_shape s, bc_tree_inputs in, int nodes, void* workspace, size_t 
   SplitPlan one = wide_plan(s, P.row_tiles, max_tiles, cus, false);
   if (!one.wide)
     one = pair_requests(P.batch, (long long)P.batch * P.hkv * P.row_tiles,
-                        SplitPlan{1, (max_tiles + 1) / 2 * 2, 8}, cus);
+                        SplitPlan{1, max_tiles, 8}, cus);
   return launch_split(P, s.dim, one, nullptr, 0, st);
 }
 

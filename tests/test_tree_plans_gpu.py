@@ -214,3 +214,84 @@ def test_pages_outside_the_pool_are_skipped(oracle):
         for workspace in (True, False):
             got = _run((k, v, bad, lengths, dq, dk, dv, par), workspace)
             G.gate(got, expected, 3e-4, f"{shape} workspace={workspace}")
+
+
+def _cuts(fix):
+    """Whether a workspace call took its units in shares or ranges: the
+    workspace's last word.  Whole units leave no partials (the records stand in
+    the final 4 KB)."""
+    k, v, pages, lengths, dq, dk, dv, par = fix
+    b, n, hq, d = dq.shape
+    shape = capi.Shape(b, hq, k.shape[2], d, pages.shape[1], k.shape[0])
+    tp, tl, tq, tdk, tdv, tpar = (G.dev(x) for x in (pages, lengths, dq, dk, dv, par))
+    out = G.nan_out((b, n, hq, d), 0)
+    ins = capi.TreeInputs(
+        capi.Inputs(None, k.data_ptr(), v.data_ptr(), tp.data_ptr(), tl.data_ptr(), None),
+        tq.data_ptr(), tdk.data_ptr(), tdv.data_ptr(), tpar.data_ptr(), out.data_ptr())
+    L = G.lib()
+    nbytes = L.bc_tree_verify_workspace_size(shape, n)
+    ws = torch.full((nbytes,), 0xff, device="cuda", dtype=torch.uint8)
+    G.check(L.bc_tree_verify_ws(shape, ins, n, ws.data_ptr(), nbytes, G.stream()), "ws call")
+    torch.cuda.synchronize()
+    taken = int(ws[-4:].view(torch.int32))
+    assert taken in (0, 1) and (taken or bool((ws[:-4096] == 0xff).all()))
+    return bool(taken)
+
+
+def _workspace(route, batch, d):
+    """Bytes of a route's partials, (max, sum) pairs, records and last word."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    rows, records = {"flat": (2 * cus * 32, cus), "wide2": (2 * cus * 64, batch),
+                     "wide4": (2 * cus * 128, batch)}[route]
+    return rows * (d * 4 + 8) + records * 8 + 4
+
+
+@pytest.mark.parametrize("route,batch,nodes,hq,hkv,d,max_pages,pool,longest,parents,cut", [
+    # Tables of 4096 tokens and more over short lengths: whole units, two
+    # requests a workgroup or one.
+    ("flat", 64, 7, 32, 8, 128, 258, 2048, 0, "random", False),
+    ("flat", 33, 8, 32, 8, 64, 800, 4096, 0, "malformed", False),
+    ("flat", 7, 16, 16, 8, 128, 1024, 2048, 200, "chain", False),
+    ("wide4", 8, 33, 32, 8, 128, 258, 0, 0, "random", False),
+    ("wide4", 1, 256, 32, 8, 128, 512, 0, 300, "malformed", False),
+    ("wide2", 16, 16, 32, 8, 128, 258, 2048, 0, "chain", False),
+    ("wide4", 16, 33, 28, 4, 64, 258, 2048, 500, "random", False),
+    ("wide2", 15, 10, 24, 4, 64, 800, 4096, 0, "random", False),  # an odd batch
+    # One request far longer than its equal part: cut.
+    ("flat", 50, 1, 32, 8, 128, 129, 2048, 2064, "random", True),      # one-tile units
+    ("flat", 64, 32, 8, 8, 128, 128, 2048, 2048, "malformed", True),   # a full draft tile
+    ("flat", 64, 31, 16, 16, 64, 250, 2048, 4000, "chain", True),      # 31 draft tokens
+    ("flat", 300, 4, 7, 1, 128, 200, 16384, 3200, "random", True),     # more requests than ranges
+    ("flat", 130, 8, 8, 2, 128, 200, 8192, 3200, "random", True),      # three windows of 64
+    ("wide2", 20, 16, 32, 8, 128, 160, 0, 2560, "random", True),
+    ("wide4", 140, 9, 8, 1, 128, 160, 0, 2560, "malformed", True),     # three windows of 64
+    ("wide2", 250, 16, 4, 1, 128, 160, 0, 2500, "random", True),       # nearly every slot
+    ("wide4", 12, 33, 28, 4, 64, 190, 2048, 3040, "random", True),
+    ("wide4", 4, 64, 32, 8, 128, 190, 2048, 3000, "chain", True),      # many shares, four rows a wave
+    ("wide2", 3, 9, 32, 8, 128, 250, 2048, 4000, "random", True),
+    # Two units per CU and more (D = 64: past two): at any length.
+    ("wide4", 8, 64, 32, 8, 128, 190, 0, 0, "malformed", True),
+    ("wide4", 12, 128, 16, 4, 64, 130, 0, 0, "chain", True),
+    ("wide4", 32, 16, 64, 4, 128, 130, 0, 0, "random", True),
+])
+def test_routes_follow_the_lengths(route, batch, nodes, hq, hkv, d, max_pages, pool, longest,
+                                   parents, cut, oracle):
+    """The table's width only says that a batch may be long."""
+    fix = _case(batch + nodes, batch, nodes, hq, hkv, d, max_pages, pool=pool, longest=longest,
+                parents=parents)
+    shape = capi.Shape(batch, hq, hkv, d, max_pages, fix[0].shape[0])
+    assert G.lib().bc_tree_verify_workspace_size(shape, nodes) == _workspace(route, batch, d)
+    assert _cuts(fix) == cut
+    _check(fix, oracle, True)
+
+
+def test_whole_units_do_not_depend_on_the_table():
+    """A short batch under a wide table over a large pool takes the tight
+    table's single pass, bit for bit, also when its neighbours are longer."""
+    k, v, pages, lengths, dq, dk, dv, par = _case(9, 64, 7, 32, 8, 128, 14)
+    tight = _run((k, v, pages, lengths, dq, dk, dv, par), True)
+    big_k, big_v = (torch.zeros((2048, *x.shape[1:]), device="cuda", dtype=x.dtype) for x in (k, v))
+    big_k[:k.shape[0]], big_v[:v.shape[0]] = k, v
+    wide = np.full((64, 512), -1, dtype=np.int32)
+    wide[:, :pages.shape[1]] = pages
+    assert np.array_equal(_run((big_k, big_v, wide, lengths, dq, dk, dv, par), True), tight)
