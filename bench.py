@@ -715,7 +715,7 @@ def main():
         print(f"[bench] C3 {results['c3_tree']}", file=sys.stderr, flush=True)
     if want("tl"):
         # A large draft tree (beyond the benchmark configs): 8 requests x 256
-        # nodes over a 2048-token shared prefix, where tree_rows_kernel shares
+        # nodes over a 2048-token shared prefix, where tree_wide_kernel shares
         # each K/V tile between four row tiles.
         results["tree_large"] = bench_tree(cx, 8, 2048, 4, with_expanded=False, nodes=256)
         print(f"[bench] tree 8 x 2048 x 256 nodes {results['tree_large']}", file=sys.stderr,

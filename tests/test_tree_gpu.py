@@ -121,13 +121,16 @@ def test_mid_batch_splits_the_prefix(oracle):
 @pytest.mark.parametrize("batch,nodes,hq,hkv,d", [(8, 128, 32, 8, 128), (8, 64, 64, 8, 64)])
 def test_large_trees_share_tiles_across_row_tiles(batch, nodes, hq, hkv, d, oracle):
     """Trees of 16 row tiles per (request, KV head) whose groups of four row
-    tiles fill the CUs (8 requests x 8 KV heads x 4 groups) take
-    tree_rows_kernel, which loads each K/V tile once for four row tiles
-    (the workspace entry point runs it too: it needs no workspace)."""
+    tiles fill the CUs (8 requests x 8 KV heads x 4 groups) load each K/V tile
+    once for four row tiles: tree_wide_kernel, and for tensors off 16-byte
+    alignment tree_rows_kernel (the workspace entry point runs them too: they
+    need no workspace)."""
     rng = np.random.default_rng(nodes + d)
     fix = oracle_np.tree_fixture(rng, batch, 300, nodes, hq=hq, hkv=hkv, d=d,
                                  parents="random")
-    _check(fix, oracle, atol=3e-4, what=f"B={batch} N={nodes} D={d}")
+    expected = _check(fix, oracle, atol=3e-4, what=f"B={batch} N={nodes} D={d}")
+    for ws in (True, False):
+        G.gate(G.tree(*fix, workspace=ws, shift=2), expected, 3e-4, f"unaligned workspace={ws}")
 
 
 def _group_fixture(rng, lengths, share, nodes=7, hq=32, hkv=8, d=128, cow_last=(),
@@ -204,8 +207,11 @@ def test_per_request_page_tables(case, oracle):
          cow_last=(10, 21)),
     # D = 64 at 8 KV heads
     dict(lengths=[300] * 40, share=[-1] + [0] * 39, hq=32, hkv=8, d=64),
-    # 16 nodes: two row tiles per (request, KV head), 1,024 units
+    # 16 nodes: two row tiles per (request, KV head); 1,024 units, whose two row
+    # tiles share K/V tiles (tree_wide_kernel), and 800, which pair requests
     dict(lengths=[300] * 64, share=[-1] + [0] * 63, nodes=16),
+    dict(lengths=[300] * 50, share=[-1] + [0] * 49, nodes=16),
+    dict(lengths=[300, 17, 0, 411, 300] * 10, share=[-1] * 50, nodes=9, d=64),
 ])
 def test_large_batches_pair_requests(case, oracle):
     """Batches with more (request, KV head) units than CUs run in one pass

@@ -2,11 +2,12 @@
 tiles, steps, parts and ranges, against the CPU oracle.
 
 tree_wide_kernel shares K/V tiles between row tiles: two or four a workgroup,
-whole or split by the batch's lengths.  tree_flat_kernel walks equal ranges of a ragged batch's
-tiles.  Which one a call takes follows from its shape, so each case's shape
-puts it on one of them; short lengths under large page tables keep the oracle
-cheap and leave shares and ranges uneven or empty.  The gate is the reference driver's
-3e-4 (src/main.cu:505-509).
+whole or split by the batch's lengths.  tree_flat_kernel walks equal ranges of a
+ragged batch's tiles.  Which kernel a call launches follows from its shape (the
+workspace's size tells which); whether its shares or ranges are taken, or whole
+units behind them, from the lengths (the workspace's last word).  Short lengths
+under large page tables keep the oracle cheap and leave shares and ranges uneven
+or empty.  The gate is the reference driver's 3e-4 (src/main.cu:505-509).
 """
 
 import numpy as np
@@ -123,6 +124,10 @@ def _check(fix, oracle, splits):
     (40, 129, 8, 8, 128, 14, False, "malformed"),
     (28, 97, 28, 4, 128, 60, False, "chain"),
     (28, 65, 32, 8, 128, 58, False, "random"),
+    # The same past 64 page ids: registers that move up by the tiles left out
+    # and are loaded again, at both head dimensions.
+    (28, 100, 28, 4, 128, 130, False, "random"),
+    (40, 200, 8, 8, 64, 130, False, "chain"),
     (64, 9, 32, 8, 64, 14, False, "random"),      # two row tiles, two workgroups per CU
     (32, 16, 32, 8, 128, 60, False, "malformed"),  # two, one workgroup per CU
     # The ancestor sets of one wave: 64 nodes, one short of them, chains and
@@ -130,7 +135,8 @@ def _check(fix, oracle, splits):
     (30, 64, 32, 8, 128, 14, False, "chain"),
     (30, 63, 32, 8, 64, 14, False, "malformed"),
     (30, 64, 32, 8, 64, 14, False, "malformed"),
-    # Split by the lengths: one long request in many shares, most in one.
+    # Tables that have room for shares, over lengths that mostly do not fill
+    # them (test_routes_follow_the_lengths has both sides).
     (20, 16, 32, 8, 128, 130, True, "random"),
     (32, 16, 32, 8, 128, 130, True, "chain"),
     (140, 9, 8, 1, 128, 130, True, "malformed"),  # requests in three windows of 64
@@ -189,12 +195,17 @@ def test_flat_ranges(batch, nodes, hq, hkv, d, max_pages, pool, longest, parents
 
 
 def test_pages_outside_the_pool_are_skipped(oracle):
-    """Ids past the pool and negative ones inside a length, on the wide and the
-    flat kernel: the result is the one without those pages' tokens."""
-    for shape in ((28, 32, 32, 8, 128, 14, None), (64, 7, 32, 8, 128, 128, 2048)):
-        batch, nodes, hq, hkv, d, max_pages, pool = shape
+    """Ids past the pool and negative ones inside a length, on the wide kernel
+    (whole units and shares), the flat one and the single pass behind them: the
+    result is the one without those pages' tokens."""
+    for shape in ((28, 32, 32, 8, 128, 14, None, 0, None), (64, 7, 32, 8, 128, 128, 2048, 0, False),
+                  (64, 7, 32, 8, 128, 128, 2048, 2048, True),
+                  (8, 64, 32, 8, 128, 190, None, 3000, True),
+                  (16, 33, 28, 4, 64, 190, None, 3000, True),
+                  (16, 16, 32, 8, 128, 130, 2048, 0, False)):
+        batch, nodes, hq, hkv, d, max_pages, pool, longest, in_shares = shape
         k, v, pages, lengths, dq, dk, dv, par = _case(5, batch, nodes, hq, hkv, d, max_pages,
-                                                      pool=pool)
+                                                      pool=pool, longest=longest)
         full = [b for b in range(batch) if lengths[b] >= 64]
         bad = pages.copy()
         cut, cut_len = np.full_like(pages, -1), lengths.copy()
@@ -205,6 +216,8 @@ def test_pages_outside_the_pool_are_skipped(oracle):
                 del row[1]
                 cut_len[b] -= 16
             cut[b, :len(row)] = row
+        if in_shares is not None:
+            assert _cuts((k, v, bad, lengths, dq, dk, dv, par)) == in_shares
         live = torch.from_numpy(np.unique(cut[cut >= 0]).astype(np.int64)).cuda()
         ren = np.full(k.shape[0], -1, dtype=np.int32)
         ren[live.cpu().numpy()] = np.arange(len(live))
