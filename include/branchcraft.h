@@ -172,7 +172,12 @@ size_t bc_tree_verify_workspace_size(bc_shape shape, int nodes);
  * bc_tree_verify_workspace_size bytes.  A null workspace, one smaller than
  * required or one not aligned to 16 bytes is ignored and the call is
  * bc_tree_verify's.  Results match bc_tree_verify within floating-point
- * reassociation (bit for bit when that call splits too). */
+ * reassociation; bit for bit when this size is at most
+ * BC_SCRATCH_SLOT_BYTES and that call gets a slot: a larger plan is cut
+ * into half as many shares where it has to fit one.
+ * Sums are FP32 throughout.  Where a batch is cut into shares of its work,
+ * their ends, and so the order of a request's sums, follow from the lengths
+ * of all its requests: a request's last bits may change with its neighbours. */
 int bc_tree_verify_ws(bc_shape shape, bc_tree_inputs in, int nodes,
                       void* workspace, size_t workspace_bytes,
                       bc_stream_t stream);
