@@ -146,7 +146,8 @@ int bc_auto_splits(bc_shape shape, int max_length, int cu_count);
  * (src/tree_attention.cu:93-105).  Shapes whose prefix splits (as
  * bc_tree_verify_ws would split it) run the split kernels with a slot of the
  * library's scratch pool (see the state note at the top), giving
- * bc_tree_verify_ws's results bit for bit; otherwise one workgroup per
+ * bc_tree_verify_ws's results bit for bit where the slot holds that call's
+ * workspace; otherwise one workgroup per
  * (request, KV head, row tile) streams the whole prefix.  Tensors that are
  * not 16-byte aligned take an element-wise single pass.
  * Rejects, as the reference: batch/Hq/Hkv < 1, Hq % Hkv != 0, dim not
