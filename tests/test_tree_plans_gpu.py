@@ -308,3 +308,46 @@ def test_whole_units_do_not_depend_on_the_table():
     wide = np.full((64, 512), -1, dtype=np.int32)
     wide[:, :pages.shape[1]] = pages
     assert np.array_equal(_run((big_k, big_v, wide, lengths, dq, dk, dv, par), True), tight)
+
+
+@pytest.mark.parametrize("batch,nodes,hq,hkv,d,max_pages,pool", [
+    (64, 7, 32, 8, 128, 128, 2048),  # ranges
+    (16, 16, 32, 8, 128, 160, 2048),  # shares of two row tiles
+    (12, 33, 28, 4, 64, 190, 2048),   # of four
+])
+def test_a_captured_call_follows_the_lengths(batch, nodes, hq, hkv, d, max_pages, pool):
+    """One graph, replayed over lengths that are cut, left whole and cut again:
+    each time the eager call's bits."""
+    k, v, pages, lengths, dq, dk, dv, par = _case(3, batch, nodes, hq, hkv, d, max_pages, pool=pool,
+                                                  longest=16 * max_pages)
+    b, n = batch, nodes
+    shape = capi.Shape(b, hq, hkv, d, max_pages, k.shape[0])
+    tp, tl, tq, tdk, tdv, tpar = (G.dev(x) for x in (pages, lengths, dq, dk, dv, par))
+    short = np.minimum(lengths, 70).astype(np.int32)
+    L = G.lib()
+    nbytes = L.bc_tree_verify_workspace_size(shape, n)
+    ws = torch.full((nbytes,), 0xff, device="cuda", dtype=torch.uint8)
+    out = G.nan_out((b, n, hq, d), 0)
+
+    def call():
+        prefix = capi.Inputs(None, k.data_ptr(), v.data_ptr(), tp.data_ptr(), tl.data_ptr(), None)
+        ins = capi.TreeInputs(prefix, tq.data_ptr(), tdk.data_ptr(), tdv.data_ptr(),
+                              tpar.data_ptr(), out.data_ptr())
+        G.check(L.bc_tree_verify_ws(shape, ins, n, ws.data_ptr(), nbytes, G.stream()), "call")
+
+    eager = {}
+    for name, lens in (("long", lengths), ("short", short)):
+        tl.copy_(torch.from_numpy(lens))
+        call()
+        torch.cuda.synchronize()
+        eager[name] = (out.clone(), int(ws[-4:].view(torch.int32)))
+    assert (eager["long"][1], eager["short"][1]) == (1, 0)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for name in ("long", "short", "long", "short", "short", "long"):
+        tl.copy_(torch.from_numpy(lengths if name == "long" else short))
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager[name][0]), name
